@@ -1,0 +1,68 @@
+"""BVH traversal at the sizes where its bookkeeping can go wrong: waves with
+one ray or one ray too many, trees of one leaf, rays with an interval that
+starts behind the origin or never ends, ties between coincident triangles,
+and stacks that move to private memory and back more than once.  Hits equal
+the brute-force loop bit for bit."""
+import numpy as np
+import pytest
+
+from test_trace_gpu import _gpu_trace, _onion
+
+pytestmark = pytest.mark.gpu
+
+
+def _soup(n, seed, copies=1):
+    """n random triangles, each present `copies` times (coincident: ties go to the lowest id)."""
+    from violet_amd import scene
+
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(-1.0, 1.0, (n, 1, 3))
+    pos = np.tile(c + rng.normal(0, 0.4, (n, 3, 3)), (copies, 1, 1)).reshape(-1, 3).astype(np.float32)
+    m = n * copies
+    return scene.Mesh(positions=pos, normals=np.tile(np.array([0, 0, 1], np.float32), (3 * m, 1)),
+                      indices=np.arange(3 * m, dtype=np.uint32).reshape(m, 3), tri_material=np.zeros(m, np.uint32),
+                      albedo=np.full((1, 3), 0.5), metallic=np.zeros(1), roughness=np.full(1, 0.5))
+
+
+def _check(vgi, mesh, rays):
+    import oracle
+    from violet_amd import scene
+
+    sc = scene.Scene(mesh)
+    g_thv, g_id = _gpu_trace(sc, rays, False)
+    o_thv, o_id = oracle.trace(32, mesh.positions, mesh.indices, rays, brute=True)
+    assert np.array_equal(g_id, o_id), f"hit ids differ on {np.mean(g_id != o_id):.3%} of rays"
+    hit = g_id != 0xFFFFFFFF
+    assert np.array_equal(g_thv[hit].view(np.uint32), o_thv[hit].astype(np.float32).view(np.uint32))
+    assert np.array_equal(_gpu_trace(sc, rays, True)[1] != 0xFFFFFFFF, hit)
+    return hit
+
+
+@pytest.mark.parametrize("n_rays", [1, 63, 64, 65, 1000])
+@pytest.mark.parametrize("n_tris,copies", [(1, 1), (2, 1), (5, 1), (3, 6), (300, 2)])
+@pytest.mark.parametrize("interval", [(5e-4, 1000.0), (-3.0, 1000.0), (0.0, np.inf), (0.5, 1.5)])
+def test_edges(vgi, n_tris, copies, n_rays, interval):
+    rng = np.random.default_rng(n_tris + n_rays)
+    o = rng.uniform(-2.0, 2.0, (n_rays, 3))
+    d = rng.uniform(-1.0, 1.0, (n_rays, 3)) - o
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    one = np.ones((n_rays, 1))
+    rays = np.concatenate([o, interval[0] * one, d, interval[1] * one], 1).astype(np.float32)
+    hit = _check(vgi, _soup(n_tris, 3, copies), rays)
+    if n_tris == 300 and n_rays == 1000:
+        assert hit.any()
+
+
+def test_stack_leaves_lds_twice(vgi):
+    """200,000 stacked quads: every box on a ray's way is hit, three children
+    stay on the stack per level, about 30 entries: two moves of eight."""
+    rng = np.random.default_rng(8)
+    m = 256
+    o = np.column_stack([rng.uniform(-0.5, 0.5, (m, 2)), np.where(rng.random(m) < 0.5, -1.0, 11.0)])
+    d = np.column_stack([rng.normal(0, 0.02, (m, 2)), np.where(o[:, 2] < 0, 1.0, -1.0)])
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.concatenate([o, np.full((m, 1), 5e-4), d, np.full((m, 1), 1000.0)], 1).astype(np.float32)
+    assert _check(vgi, _onion(200_000, 4), rays).all()
+    # any hit from inside the pile: early exits while entries wait in private memory
+    rays[:, 2] = rng.uniform(0.0, 10.0, m)
+    _check(vgi, _onion(200_000, 4), rays)

@@ -252,7 +252,7 @@ extern "C" vgi_status vgi_batch_add_passes(vgi_batch* b, const vgi_scene* scene,
         if (persistent_groups(b, o) == 0 && tiles > b->grid_bound[s]) b->grid_bound[s] = tiles;
     }
     // 3. upload + fused launches
-    const size_t lds = traversal_lds_bytes(scene_view(scene));
+    const size_t lds = traversal_lds_bytes();
     if (!b->cfg.use_graph) {
         vgi_status r = issue_frame(b, a, storage, lds, st, false, true);
         if (r != VGI_OK) return r;

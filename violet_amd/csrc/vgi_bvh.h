@@ -99,11 +99,14 @@ constexpr float kRayTMin = 0.0005f;  // raytrace.inc.hlsl:39,70
 constexpr float kRayTMax = 1000.0f;  // raytrace.inc.hlsl:40,71
 constexpr int kBvhMaxDepth = 64;     // binary build depth bound (the 4-wide tree is shallower)
 
-// Traversal stack: the bottom kLdsStackEntries entries of each lane live in
-// LDS, deeper ones in private (scratch) memory.  A one-wave workgroup with a
-// 4 KiB stack leaves LDS for more resident waves than the registers allow,
-// and the scratch part is touched only by rays whose stack grows past 16.
-constexpr uint32_t kLdsStackEntries = 16;
+// Traversal stack: kLdsStackEntries entries of each lane live in LDS (two of
+// them sentinels, four the room a node step writes before it pops), older
+// ones in private (scratch) memory, moved kSpillEntries at a time.  5 KiB per
+// one-wave workgroup is the most that leaves LDS (160 KiB per CU) for 32
+// resident waves; the scratch part is touched only by rays that hold more
+// than 14 entries.
+constexpr uint32_t kLdsStackEntries = 20;
+constexpr int kSpillEntries = 8;
 constexpr uint32_t kStackMaxEntries = 3 * kBvhMaxDepth;  // 3 far children per 4-wide level
 
 // Register budget of the per-pixel ray-tracing kernels, as waves per SIMD:
@@ -129,11 +132,8 @@ struct HostScene {
 };
 vgi_status build_scene_host(const vgi_scene_desc* desc, HostScene& out);
 
-// Dynamic LDS bytes of a 64-lane traversal stack for this scene.
-inline size_t traversal_lds_bytes(const SceneView& s) {
-    const uint32_t e = s.stack_depth < kLdsStackEntries ? s.stack_depth : kLdsStackEntries;
-    return (size_t)e * 64u * sizeof(int32_t);
-}
+// Dynamic LDS bytes of a 64-lane traversal stack.
+inline size_t traversal_lds_bytes() { return (size_t)kLdsStackEntries * 64u * sizeof(int32_t); }
 
 struct Hit {
     float t;

@@ -285,9 +285,9 @@ extern "C" vgi_status vgi_pass_raytraced_shadow(const vgi_frame_params* fp, cons
     sv.counters = trace_counters();
     const dim3 g = tile_grid(io->width, io->height);
     if (sv.counters)
-        hipLaunchKernelGGL(k_raytraced_shadow<true>, g, dim3(64), traversal_lds_bytes(sv), st, f, sv, *io);
+        hipLaunchKernelGGL(k_raytraced_shadow<true>, g, dim3(64), traversal_lds_bytes(), st, f, sv, *io);
     else
-        hipLaunchKernelGGL(k_raytraced_shadow<false>, g, dim3(64), traversal_lds_bytes(sv), st, f, sv, *io);
+        hipLaunchKernelGGL(k_raytraced_shadow<false>, g, dim3(64), traversal_lds_bytes(), st, f, sv, *io);
     trace_stats_collect("raytraced_shadow", st);
     return check_launch("k_raytraced_shadow");
 }

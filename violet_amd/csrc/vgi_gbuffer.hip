@@ -148,9 +148,9 @@ extern "C" vgi_status vgi_pass_gbuffer_primary(const vgi_frame_params* fp, const
     sv.counters = trace_counters();
     const dim3 g = tile8_grid(io->width, io->height);
     if (sv.counters)
-        hipLaunchKernelGGL(k_gbuffer<true>, g, dim3(64), traversal_lds_bytes(sv), st, f, sv, *io);
+        hipLaunchKernelGGL(k_gbuffer<true>, g, dim3(64), traversal_lds_bytes(), st, f, sv, *io);
     else
-        hipLaunchKernelGGL(k_gbuffer<false>, g, dim3(64), traversal_lds_bytes(sv), st, f, sv, *io);
+        hipLaunchKernelGGL(k_gbuffer<false>, g, dim3(64), traversal_lds_bytes(), st, f, sv, *io);
     trace_stats_collect("gbuffer_primary", st);
     return check_launch("k_gbuffer");
 }

@@ -389,7 +389,7 @@ static FrameParams to_fp(const vgi_frame_params* fp) {
 // and the instrumented build when traversal statistics are on.
 #define VGI_DISPATCH_STORAGE(mode, kernel, grid, ...)                                                      \
     do {                                                                                                   \
-        const size_t lds_ = traversal_lds_bytes(t.scene);                                                  \
+        const size_t lds_ = traversal_lds_bytes();                                                  \
         const bool f32_ = (mode) == VGI_STORAGE_F32;                                                       \
         if (t.scene.counters) {                                                                            \
             if (f32_)                                                                                      \

@@ -43,9 +43,9 @@ extern "C" vgi_status vgi_trace_rays(const vgi_scene* scene, const float* rays, 
     sv.counters = trace_counters();
     const dim3 g((num_rays + 63) / 64);
     if (sv.counters)
-        hipLaunchKernelGGL(k_trace_rays<true>, g, dim3(64), traversal_lds_bytes(sv), st, sv, rays, num_rays, any_hit, hits);
+        hipLaunchKernelGGL(k_trace_rays<true>, g, dim3(64), traversal_lds_bytes(), st, sv, rays, num_rays, any_hit, hits);
     else
-        hipLaunchKernelGGL(k_trace_rays<false>, g, dim3(64), traversal_lds_bytes(sv), st, sv, rays, num_rays, any_hit, hits);
+        hipLaunchKernelGGL(k_trace_rays<false>, g, dim3(64), traversal_lds_bytes(), st, sv, rays, num_rays, any_hit, hits);
     trace_stats_collect(name, st);
     return check_launch("k_trace_rays");
 }

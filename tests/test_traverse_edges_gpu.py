@@ -66,3 +66,15 @@ def test_stack_leaves_lds_twice(vgi):
     # any hit from inside the pile: early exits while entries wait in private memory
     rays[:, 2] = rng.uniform(0.0, 10.0, m)
     _check(vgi, _onion(200_000, 4), rays)
+
+
+@pytest.mark.parametrize("n_tris", [16384, 16385, 40000])
+def test_scene_built_in_pieces(vgi, n_tris):
+    """Scenes at and past the size from which subtrees are built apart and put together."""
+    rng = np.random.default_rng(n_tris)
+    m = 300
+    o = rng.uniform(-2.0, 2.0, (m, 3))
+    d = rng.uniform(-1.0, 1.0, (m, 3)) - o
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.concatenate([o, np.full((m, 1), 5e-4), d, np.full((m, 1), 1000.0)], 1).astype(np.float32)
+    assert _check(vgi, _soup(n_tris, 5), rays).any()

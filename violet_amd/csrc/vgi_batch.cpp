@@ -40,9 +40,9 @@ static const char* kind_name(int kind) {
     static const char* n[kPassKindCount] = {
         "batch_clear",           "batch_gbuffer_primary",      "batch_hash_grid_decay",
         "batch_hash_grid_query_select", "batch_hash_grid_query_compact", "batch_hash_grid_raygen",
-        "batch_ind_diff_sample_gen", "batch_ind_diff_sample_validate", "batch_raytraced_ao_gen",
+        "batch_ind_spec_sample", "batch_ind_diff_sample", "batch_raytraced_ao_gen",
         "batch_raytraced_ao_filter", "batch_ind_diff_temporal_resample", "batch_ind_diff_spatial_resample",
-        "batch_ind_spec_sample_gen", "batch_ind_spec_sample_validate", "batch_ind_spec_temporal_resample",
+        "batch_ind_spec_temporal_resample",
         "batch_ind_spec_spatial_resample", "batch_denoise_temporal", "batch_denoise_disocclusion_fix",
         "batch_denoise_fast_history_clamp", "batch_denoise_spatial_fallback", "batch_denoise_atrous",
         "batch_raytraced_shadow", "batch_final_lighting", "batch_temporal_aa",
@@ -66,7 +66,7 @@ struct vgi_batch {
     hipEvent_t ev_in = nullptr;
     // second lane (concurrent_lanes): independent slot chains beside the main stream
     hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_cross = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     hipGraphExec_t exec[2] = {nullptr, nullptr};
     uint32_t key_storage[2] = {0, 0};
     uint32_t key_shape[2][2] = {{0, 0}, {0, 0}};  // launch shapes (vgi_tuning) the graph was captured with
@@ -89,7 +89,6 @@ struct vgi_batch {
         if (ev_in) (void)hipEventDestroy(ev_in);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
-        if (ev_cross) (void)hipEventDestroy(ev_cross);
         if (side) (void)hipStreamDestroy(side);
         if (cap) (void)hipStreamDestroy(cap);
     }
@@ -150,7 +149,6 @@ extern "C" vgi_status vgi_batch_create(const vgi_batch_config* cfg, vgi_batch** 
     const unsigned lane_ev = hipEventDisableTiming | hipEventDisableSystemFence;
     if (e == hipSuccess && c.concurrent_lanes) e = hipEventCreateWithFlags(&b->ev_fork, lane_ev);
     if (e == hipSuccess && c.concurrent_lanes) e = hipEventCreateWithFlags(&b->ev_join, lane_ev);
-    if (e == hipSuccess && c.concurrent_lanes) e = hipEventCreateWithFlags(&b->ev_cross, lane_ev);
     if (e != hipSuccess) {
         delete b;
         return check_hip(e, "vgi_batch_create");
@@ -195,7 +193,6 @@ static vgi_status issue_slots(vgi_batch* b, int a, uint32_t storage, size_t lds,
         } else {
             r = o->launch((const char*)b->dev[a] + b->offsets[s], storage, groups_for(b, s, o), o->trace ? lds : 0, st);
         }
-        if (r == VGI_OK) r = lanes.leave(s, st);
         if (r != VGI_OK) return r;
     }
     return VGI_OK;
@@ -208,7 +205,6 @@ static vgi_status issue_frame(vgi_batch* b, int a, uint32_t storage, size_t lds,
     lanes.side = b->side;
     lanes.ev_fork = b->ev_fork;
     lanes.ev_join = b->ev_join;
-    lanes.ev_cross = b->ev_cross;
     vgi_status r = issue_slots(b, a, storage, lds, lanes, all_slots, profile);
     vgi_status j = lanes.finish();
     return r != VGI_OK ? r : j;

@@ -23,33 +23,18 @@ vgi_status Lanes::enter(int slot, hipStream_t& st) {
         VGI_TRY_HIP(hipEventRecord(ev_fork, main));
         VGI_TRY_HIP(hipStreamWaitEvent(side, ev_fork, 0));
         phase = ph;
-        cross_pending = false;
     }
     if (slot_lane(slot)) {
         st = side;
         side_work = true;
     }
-    if (slot_waits(slot) && cross_pending && cross_from != st) {
-        VGI_TRY_HIP(hipStreamWaitEvent(st, ev_cross, 0));
-        cross_pending = false;
-    }
-    return VGI_OK;
-}
-
-vgi_status Lanes::leave(int slot, hipStream_t st) {
-    if (!side || !ev_cross || !slot_signals(slot)) return VGI_OK;
-    VGI_TRY_HIP(hipEventRecord(ev_cross, st));
-    cross_from = st;  // may be the null stream: cross_pending says that ev_cross is set
-    cross_pending = true;
     return VGI_OK;
 }
 
 vgi_status DirectSink::submit(int slot, const PassRec& r) {
     hipStream_t st;
-    vgi_status e = lanes.enter(slot, st);
-    if (e == VGI_OK) e = launch(r, st);
-    if (e == VGI_OK) e = lanes.leave(slot, st);
-    return e;
+    const vgi_status e = lanes.enter(slot, st);
+    return e == VGI_OK ? launch(r, st) : e;
 }
 
 vgi_status DirectSink::launch(const PassRec& r, hipStream_t st) {
@@ -72,8 +57,8 @@ vgi_status DirectSink::launch(const PassRec& r, hipStream_t st) {
         case kPassHgCompactOrdered: return vgi_pass_hash_grid_query_compact_ordered(&r.io.hg_ocompact, s);
         case kPassHgRaygenOrdered:
             return vgi_pass_hash_grid_raygen_ordered(&r.fp, &r.tr, &r.io.hg_oraygen, &r.pc.frame_hash, s);
-        case kPassDiffGen: return vgi_pass_ind_diff_sample_gen(&r.fp, &r.tr, &r.io.diff_gen, &r.pc.sample_gen, s);
-        case kPassDiffValidate: return vgi_pass_ind_diff_sample_validate(&r.fp, &r.tr, &r.io.diff_validate, s);
+        case kPassSampleSpec:
+        case kPassSampleDiff: return launch_sample_rays(r, st);
         case kPassAoGen: return vgi_pass_raytraced_ao_gen(&r.fp, &r.io.ao_gen, &r.pc.ao_gen, s);
         case kPassAoFilter: return vgi_pass_raytraced_ao_filter(&r.io.ao_filter, s);
         case kPassDiffTemporal:
@@ -81,8 +66,6 @@ vgi_status DirectSink::launch(const PassRec& r, hipStream_t st) {
                                         r.diff_taps_gbuffer, st);
         case kPassDiffSpatial:
             return launch_diff_spatial(&r.fp, &r.io.diff_spatial, &r.pc.diff_spatial, &r.resample, r.diff_taps, st);
-        case kPassSpecGen: return vgi_pass_ind_spec_sample_gen(&r.fp, &r.tr, &r.io.spec_gen, &r.pc.sample_gen, s);
-        case kPassSpecValidate: return vgi_pass_ind_spec_sample_validate(&r.fp, &r.tr, &r.io.spec_validate, s);
         case kPassSpecTemporal:
             return vgi_pass_ind_spec_temporal_resample(&r.fp, &r.io.spec_temporal, &r.pc.spec_temporal, &r.resample, s);
         case kPassSpecSpatial:

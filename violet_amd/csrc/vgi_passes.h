@@ -22,14 +22,12 @@ enum PassKind : int {
     kPassHgSelect,
     kPassHgCompact,
     kPassHgRaygen,
-    kPassDiffGen,
-    kPassDiffValidate,
+    kPassSampleSpec,       // one lobe's sample generation and validation passes, in one launch
+    kPassSampleDiff,
     kPassAoGen,
     kPassAoFilter,
     kPassDiffTemporal,
     kPassDiffSpatial,
-    kPassSpecGen,
-    kPassSpecValidate,
     kPassSpecTemporal,
     kPassSpecSpatial,
     kPassDenTemporal,
@@ -63,14 +61,12 @@ enum Slot : int {
     kSlotClearNextCounter,
     kSlotHgRaygen,
     kSlotHgRaygenOrdered,
-    kSlotSpecValidate,  // issued ahead of the diffuse passes (see slot_lane)
-    kSlotDiffGen,
-    kSlotDiffValidate,
+    kSlotSampleSpec,  // issued ahead of the diffuse passes
+    kSlotSampleDiff,
     kSlotAoGen,
     kSlotAoFilter,
     kSlotDiffTemporal,
     kSlotDiffSpatial,
-    kSlotSpecGen,
     kSlotSpecTemporal,
     kSlotSpecSpatial,
     kSlotDenClearFastDiff,
@@ -92,13 +88,29 @@ inline int slot_kind(int slot) {
         kPassGBuffer,      kPassClear,        kPassClear,         kPassClear,       kPassClear,       kPassHgDecay,
         kPassClear,        kPassHgSelect,     kPassClear,         kPassHgSelectOrdered, kPassClear, kPassHgCompact,
         kPassHgCompactOrdered, kPassClear,    kPassHgRaygen,      kPassHgRaygenOrdered,
-        kPassSpecValidate, kPassDiffGen,      kPassDiffValidate,  kPassAoGen,
-        kPassAoFilter,     kPassDiffTemporal, kPassDiffSpatial,   kPassSpecGen,     kPassSpecTemporal,
+        kPassSampleSpec,   kPassSampleDiff,   kPassAoGen,        kPassAoFilter,      kPassDiffTemporal, kPassDiffSpatial, kPassSpecTemporal,
         kPassSpecSpatial,  kPassClear,        kPassClear,         kPassDenTemporal, kPassDenDisocclusion,
         kPassDenFastClamp, kPassDenFallback,  kPassDenAtrous,     kPassDenAtrous,   kPassDenAtrous,
         kPassDenAtrous,    kPassDenAtrous,    kPassShadow,        kPassFinalLighting, kPassTemporalAA};
     return k[slot];
 }
+
+// The ray passes of one view, frame and lobe that one launch runs
+// (k_sample_rays).  None of them reads what another writes: they share the
+// frame parameters, the trace resources and the image size, and append to
+// one query buffer.
+enum SamplePass : uint32_t { kSampleSpecValidate, kSampleDiffGen, kSampleDiffValidate, kSampleSpecGen, kSamplePassCount };
+struct SampleSet {
+    uint32_t count;
+    uint32_t pass[kSamplePassCount];  // SamplePass of each of the `count` parts
+    vgi_ind_spec_sample_validate_io spec_validate;
+    vgi_ind_diff_sample_gen_io diff_gen;
+    vgi_ind_diff_sample_validate_io diff_validate;
+    vgi_ind_spec_sample_gen_io spec_gen;
+    vgi_pc_sample_gen diff_pc, spec_pc;
+    void add(SamplePass p) { pass[count++] = p; }
+    bool spec() const { return pass[0] == kSampleSpecValidate || pass[0] == kSampleSpecGen; }
+};
 
 struct PassRec {
     int kind;
@@ -114,14 +126,11 @@ struct PassRec {
         vgi_hash_grid_ordered_select_io hg_oselect;
         vgi_hash_grid_ordered_compact_io hg_ocompact;
         vgi_hash_grid_ordered_raygen_io hg_oraygen;
-        vgi_ind_diff_sample_gen_io diff_gen;
-        vgi_ind_diff_sample_validate_io diff_validate;
+        SampleSet sample;
         vgi_ao_gen_io ao_gen;
         vgi_ao_filter_io ao_filter;
         vgi_ind_diff_temporal_io diff_temporal;
         vgi_ind_diff_spatial_io diff_spatial;
-        vgi_ind_spec_sample_gen_io spec_gen;
-        vgi_ind_spec_sample_validate_io spec_validate;
         vgi_ind_spec_temporal_io spec_temporal;
         vgi_ind_spec_spatial_io spec_spatial;
         vgi_denoise_temporal_io den_temporal;
@@ -134,7 +143,6 @@ struct PassRec {
     } io;
     union {
         vgi_pc_frame_hash frame_hash;
-        vgi_pc_sample_gen sample_gen;
         vgi_pc_ao_gen ao_gen;
         vgi_pc_ind_diff_temporal diff_temporal;
         vgi_pc_ind_diff_spatial diff_spatial;
@@ -188,50 +196,46 @@ struct PassSink {
 // sampling and resampling (lane 1; both read the G-buffer and the updated
 // cache, and only append to the shared query buffer); phase 2: denoiser
 // (lane 0) beside the sun shadow mask (lane 1: it reads the depth only);
-// phase 3: final lighting, then temporal AA.  The specular validation re-
-// traces last frame's samples and needs nothing of this frame's specular
-// generation, so it runs at the head of lane 0, which balances the two
-// lanes' ray tracing; the specular temporal pass waits for it (a cross-lane
-// event, slot_signals / slot_waits).
+// phase 3: final lighting, then temporal AA.
+//
+// A ray pass ends with a few waves that hold its longest rays, about 100 us
+// whatever its size.  So the specular validation, which re-traces last
+// frame's samples and needs nothing of this frame's, shares the launch of the
+// specular generation instead of a place ahead of the diffuse one: the
+// phase's rays end once.  Two lanes rather than one launch of all three:
+// the diffuse resampling then overlaps the specular rays (1080p frame 1697 us
+// with one launch).
 inline int slot_phase(int slot) {
-    return slot < kSlotSpecValidate ? 0 : slot < kSlotDenClearFastDiff ? 1 : slot < kSlotFinalLighting ? 2 : 3;
+    return slot < kSlotSampleSpec ? 0 : slot < kSlotDenClearFastDiff ? 1 : slot < kSlotFinalLighting ? 2 : 3;
 }
 inline int slot_lane(int slot) {
-    return (slot >= kSlotClearHgStorage && slot <= kSlotHgRaygenOrdered) || (slot >= kSlotSpecGen && slot <= kSlotSpecSpatial) ||
-           slot == kSlotShadow;
+    return (slot >= kSlotClearHgStorage && slot <= kSlotSampleSpec) || slot == kSlotSpecTemporal ||
+           slot == kSlotSpecSpatial || slot == kSlotShadow;
 }
-inline bool slot_signals(int slot) { return slot == kSlotSpecValidate; }
-inline bool slot_waits(int slot) { return slot == kSlotSpecTemporal; }
 
 // The streams of a frame's slots, issued in slot order.  Without a side
 // stream every slot runs on `main`.  With one, lane-1 slots go to `side`:
 // entering a phase joins the side stream into the main one (if it has work)
 // and forks it again from the main stream, so a lane-1 slot waits for every
 // earlier phase and for nothing else; finish() joins it back at the end.
-// leave() after a signalling slot records ev_cross on its stream, and a
-// waiting slot of the same phase on the other lane waits for it.  Works the
-// same under stream capture (the side stream joins the capture).
+// Works the same under stream capture (the side stream joins the capture).
 struct Lanes {
     hipStream_t main = nullptr, side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_cross = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int phase = -1;
     bool side_work = false;
-    bool cross_pending = false;        // ev_cross was recorded in this phase
-    hipStream_t cross_from = nullptr;  // the stream it was recorded on
     vgi_status enter(int slot, hipStream_t& st);
-    vgi_status leave(int slot, hipStream_t st);
     vgi_status finish();
 };
 
 // Launches each record at once through its C entry point.
 struct DirectSink : PassSink {
     explicit DirectSink(hipStream_t s) { lanes.main = s; }
-    DirectSink(hipStream_t s, hipStream_t side, hipEvent_t fork, hipEvent_t join, hipEvent_t cross) {
+    DirectSink(hipStream_t s, hipStream_t side, hipEvent_t fork, hipEvent_t join) {
         lanes.main = s;
         lanes.side = side;
         lanes.ev_fork = fork;
         lanes.ev_join = join;
-        lanes.ev_cross = cross;
     }
     vgi_status submit(int slot, const PassRec& r) override;
     vgi_status finish() { return lanes.finish(); }
@@ -240,6 +244,9 @@ struct DirectSink : PassSink {
    private:
     static vgi_status launch(const PassRec& r, hipStream_t st);
 };
+
+// The launch of a kPassSampleSpec or kPassSampleDiff record (vgi_sample.hip).
+vgi_status launch_sample_rays(const PassRec& r, hipStream_t st);
 
 // Keeps the records of one view's frame by slot.
 struct RecordSink : PassSink {

@@ -60,12 +60,11 @@ struct vgi_renderer {
 
     // second lane of add_passes (concurrent_lanes): stream + fork/join events
     hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_cross = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     ~vgi_renderer() {
         if (den) vgi_denoiser_destroy(den);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
-        if (ev_cross) (void)hipEventDestroy(ev_cross);
         if (side) (void)hipStreamDestroy(side);
     }
     std::vector<std::pair<std::string, DevBuf*>> images() {
@@ -221,7 +220,6 @@ extern "C" vgi_status vgi_renderer_create(uint32_t width, uint32_t height, const
         const unsigned lane_ev = hipEventDisableTiming | hipEventDisableSystemFence;
         if (e == hipSuccess) e = hipEventCreateWithFlags(&r->ev_fork, lane_ev);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&r->ev_join, lane_ev);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&r->ev_cross, lane_ev);
         if (e != hipSuccess) st = check_hip(e, "vgi_renderer_create: side stream");
     }
     if (st != VGI_OK) {
@@ -358,36 +356,48 @@ vgi_status vgi_renderer_plan(vgi_renderer* r, const vgi_scene* scene, const vgi_
         hg_updated = true;
     }
 
-    // Specular sample validate (:722-737): issued first, it re-traces last
-    // frame's specular samples and is independent of this frame's passes
-    // up to the specular temporal resample
+    // The frame's rays, a launch per lobe: specular sample validate (:722-737,
+    // last frame's specular samples traced again) and gen (:685-701);
+    // indirect diffuse sample gen or validation (:436-513).  The frame's
+    // random numbers keep the reference's order.
     const bool has_prev_spec = r->has_prev_ind_spec;
-    if (r->cfg.ind_spec_validate && has_prev_depth && has_prev_ind_diff && has_prev_spec) {
-        PassRec v = make_rec(kPassSpecValidate, fp);
-        v.tr = trace_res(r, scene, true);
-        v.io.spec_validate = vgi_ind_spec_sample_validate_io{w, h, S, r->spec_rsv[p].as<uint32_t>(),
-                                                             r->spec_hitpos[p].as<float>(), r->spec_rad[p].p};
-        CALL(sink.submit(kSlotSpecValidate, v));
-    }
-
-    // Indirect diffuse: sample gen or validation (:436-513)
     const bool has_prev_diff_rsv = r->has_prev_diffuse_reservoir;
     const bool validation = has_prev_depth && has_prev_diff_rsv && ((frame_index & 3u) == 0u) && r->cfg.ind_diff_validate;
     const uint32_t has_new_sample = validation ? 0u : 1u;
     const bool trace_prev = has_prev_depth && has_prev_ind_diff;
-    if (!validation) {
-        PassRec g = make_rec(kPassDiffGen, fp);
+    const uint32_t diff_gen_rand = validation ? 0u : frame_rand_next(frame_rand);
+    const uint32_t diff_temporal_rand = frame_rand_next(frame_rand);
+    const uint32_t diff_spatial_rand = frame_rand_next(frame_rand);
+    {
+        PassRec g = make_rec(kPassSampleSpec, fp);
         g.tr = trace_res(r, scene, trace_prev);
-        g.io.diff_gen = vgi_ind_diff_sample_gen_io{w, h, S, r->gbuffer[c].as<uint32_t>(), r->depth[c].as<float>(),
-                                                   r->dnew_hit.as<uint32_t>(), r->dnew_rad.p};
-        g.pc.sample_gen = vgi_pc_sample_gen{frame_rand_next(frame_rand), trace_prev ? 1u : 0u};
-        CALL(sink.submit(kSlotDiffGen, g));
-    } else {
-        PassRec v = make_rec(kPassDiffValidate, fp);
-        v.tr = trace_res(r, scene, true);
-        v.io.diff_validate = vgi_ind_diff_sample_validate_io{w, h, S, r->depth[p].as<float>(), r->dsp_rsv[p].as<uint32_t>(),
-                                                             r->dsp_hit[p].as<uint32_t>(), r->dsp_rad[p].p};
-        CALL(sink.submit(kSlotDiffValidate, v));
+        SampleSet& a = g.io.sample;
+        if (r->cfg.ind_spec_validate && trace_prev && has_prev_spec) {
+            a.spec_validate = vgi_ind_spec_sample_validate_io{w, h, S, r->spec_rsv[p].as<uint32_t>(),
+                                                              r->spec_hitpos[p].as<float>(), r->spec_rad[p].p};
+            a.add(kSampleSpecValidate);
+        }
+        a.spec_gen = vgi_ind_spec_sample_gen_io{w, h, S, r->gbuffer[c].as<uint32_t>(), r->depth[c].as<float>(),
+                                                r->spec_hitpos[c].as<float>(), r->spec_rad[c].p};
+        a.spec_pc = vgi_pc_sample_gen{frame_rand_next(frame_rand), trace_prev ? 1u : 0u};
+        a.add(kSampleSpecGen);
+        CALL(sink.submit(kSlotSampleSpec, g));
+    }
+    {
+        PassRec g = make_rec(kPassSampleDiff, fp);
+        g.tr = trace_res(r, scene, trace_prev || validation);
+        SampleSet& a = g.io.sample;
+        if (!validation) {
+            a.diff_gen = vgi_ind_diff_sample_gen_io{w, h, S, r->gbuffer[c].as<uint32_t>(), r->depth[c].as<float>(),
+                                                    r->dnew_hit.as<uint32_t>(), r->dnew_rad.p};
+            a.diff_pc = vgi_pc_sample_gen{diff_gen_rand, trace_prev ? 1u : 0u};
+            a.add(kSampleDiffGen);
+        } else {
+            a.diff_validate = vgi_ind_diff_sample_validate_io{w, h, S, r->depth[p].as<float>(), r->dsp_rsv[p].as<uint32_t>(),
+                                                              r->dsp_hit[p].as<uint32_t>(), r->dsp_rad[p].p};
+            a.add(kSampleDiffValidate);
+        }
+        CALL(sink.submit(kSlotSampleDiff, g));
     }
 
     // AO gen + filter (:515-563)
@@ -414,7 +424,7 @@ vgi_status vgi_renderer_plan(vgi_renderer* r, const vgi_scene* scene, const vgi_
                                     r->dtm_rsv.as<uint32_t>(), r->dtm_hit.as<uint32_t>(), r->dtm_rad.p};
         // has_prev_frame = has_prev_diffuse_reservoir (restir_renderer.rs:605); the
         // previous depth exists whenever the previous reservoir does
-        t.pc.diff_temporal = vgi_pc_ind_diff_temporal{frame_rand_next(frame_rand), (has_prev_diff_rsv && has_prev_depth) ? 1u : 0u,
+        t.pc.diff_temporal = vgi_pc_ind_diff_temporal{diff_temporal_rand, (has_prev_diff_rsv && has_prev_depth) ? 1u : 0u,
                                     has_new_sample};
         t.resample = resample_params(r);
         t.diff_taps = r->dtaps.as<DiffTap>();
@@ -425,21 +435,13 @@ vgi_status vgi_renderer_plan(vgi_renderer* r, const vgi_scene* scene, const vgi_
                                     r->dtm_rsv.as<uint32_t>(), r->dtm_hit.as<uint32_t>(), r->dtm_rad.p,
                                     r->dsp_rsv[c].as<uint32_t>(), r->dsp_hit[c].as<uint32_t>(), r->dsp_rad[c].p,
                                     r->diff_light[c].p};
-        sp.pc.diff_spatial = vgi_pc_ind_diff_spatial{frame_rand_next(frame_rand)};
+        sp.pc.diff_spatial = vgi_pc_ind_diff_spatial{diff_spatial_rand};
         sp.resample = resample_params(r);
         sp.diff_taps = r->dtaps.as<DiffTap>();
         CALL(sink.submit(kSlotDiffSpatial, sp));
     }
 
-    // Specular sample gen (:685-701), temporal (:743-761), spatial (:770-784)
-    {
-        PassRec g = make_rec(kPassSpecGen, fp);
-        g.tr = trace_res(r, scene, trace_prev);
-        g.io.spec_gen = vgi_ind_spec_sample_gen_io{w, h, S, r->gbuffer[c].as<uint32_t>(), r->depth[c].as<float>(),
-                                                   r->spec_hitpos[c].as<float>(), r->spec_rad[c].p};
-        g.pc.sample_gen = vgi_pc_sample_gen{frame_rand_next(frame_rand), trace_prev ? 1u : 0u};
-        CALL(sink.submit(kSlotSpecGen, g));
-    }
+    // Specular temporal (:743-761), spatial (:770-784)
     {
         const bool hp = has_prev_depth && has_prev_spec && has_prev_gbuffer;
         PassRec t = make_rec(kPassSpecTemporal, fp);
@@ -528,7 +530,7 @@ uint32_t vgi_renderer_storage(const vgi_renderer* r) { return r->cfg.storage; }
 extern "C" vgi_status vgi_renderer_add_passes(vgi_renderer* r, const vgi_scene* scene, const vgi_frame_params* fp,
                                               uint32_t frame_index, vgi_renderer_output* out, void* stream) {
     VGI_REQUIRE(r, "vgi_renderer_add_passes: null renderer");
-    DirectSink sink((hipStream_t)stream, r->side, r->ev_fork, r->ev_join, r->ev_cross);
+    DirectSink sink((hipStream_t)stream, r->side, r->ev_fork, r->ev_join);
     vgi_status s = vgi_renderer_plan(r, scene, fp, frame_index, out, sink);
     vgi_status j = sink.finish();
     return s != VGI_OK ? s : j;

@@ -88,10 +88,14 @@ void drain_locked() {
 }
 }  // namespace
 
-ProfScope::ProfScope(const char* name, hipStream_t s, double bytes) {
+bool profiling_pass(const char* name) {
     std::lock_guard<std::mutex> lk(g_prof_mu);
-    if (!g_prof_on) return;
-    if (!g_prof_only.empty() && g_prof_only != name) return;
+    return g_prof_on && (g_prof_only.empty() || g_prof_only == name);
+}
+
+ProfScope::ProfScope(const char* name, hipStream_t s, double bytes) {
+    if (!profiling_pass(name)) return;
+    std::lock_guard<std::mutex> lk(g_prof_mu);
     a_ = take_event();
     if (!a_) return;
     if (hipEventRecord(a_, s) != hipSuccess) {

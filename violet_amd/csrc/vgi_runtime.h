@@ -58,6 +58,9 @@ class ProfScope {
     double bytes_ = 0;
 };
 
+// Whether a ProfScope of this name would record now.
+bool profiling_pass(const char* name);
+
 // Traversal statistics: kTraceCounterSlots slots of {closest rays, any-hit
 // rays, interior nodes, triangles}, spread over slots to limit contention.
 constexpr int kTraceCounterSlots = 64;

@@ -1,11 +1,11 @@
 /*
  * vgi_sample.hip — the radiance-tracing passes of the ReSTIR GI path:
  *
- *   k_diff_sample_gen      restir/ind_diff_sample_gen.hlsl:25-67
- *   k_diff_sample_validate restir/ind_diff_sample_validate.hlsl:90-145
- *   k_spec_sample_gen      restir/ind_spec_sample_gen.hlsl:28-128
- *   k_spec_sample_validate restir/ind_spec_sample_validate.hlsl:144-191
- *   k_hash_grid_raygen     restir/hash_grid_raygen.hlsl:141-204
+ *   k_sample_rays       restir/ind_diff_sample_gen.hlsl:25-67,
+ *                       restir/ind_diff_sample_validate.hlsl:90-145,
+ *                       restir/ind_spec_sample_gen.hlsl:28-128,
+ *                       restir/ind_spec_sample_validate.hlsl:144-191
+ *   k_hash_grid_raygen  restir/hash_grid_raygen.hlsl:141-204
  *
  * One lane per pixel (or per compacted cache query, 16 per wave).  Each lane traces one
  * GI ray plus one sun shadow ray through the LDS-stack traversal.  Pixels
@@ -29,7 +29,7 @@ __device__ __forceinline__ f3 position_biased(const float* m, uint32_t px, uint3
 // Each sample pass is a pair of functions around trace_radiance: gen_px()
 // turns a pixel into its GI ray (or writes the outputs of a pixel without
 // one and returns false) and finish_px() writes the outputs of the traced
-// sample; sample_pixel() runs the pair for one lane per pixel.
+// sample; k_sample_rays runs the pair for one lane per pixel.
 template <class S>
 struct DiffGenPass {
     const FrameParams& fp;
@@ -63,38 +63,6 @@ struct DiffGenPass {
         S::st3(io.rw_hit_radiance_texture, i, r.radiance);
     }
 };
-
-// One lane per pixel of tile (bx_, by_): 8x8 pixels in 2x2 quads, or rows of
-// rt.tile_w pixels (16 x 4, 32 x 2); the shape is a launch parameter
-// (vgi_tuning) and does not change any pixel's result.
-template <class P, class S, bool kCount>
-__device__ __forceinline__ void sample_pixel(const P& p, const TraceRes& rt, const FrameParams& fp, bool has_prev,
-                                             uint32_t bx_, uint32_t by_) {
-    VGI_TRAVERSAL_STACK(stack);
-    uint32_t px, py;
-    if (rt.tile_w == 8u) {
-        quad_tile_pixel_at<8>(bx_, by_, px, py);
-    } else {
-        const uint32_t lane = threadIdx.x & 63u, sh = rt.tile_w == 16u ? 4u : 5u;
-        px = (bx_ << sh) + (lane & (rt.tile_w - 1u));
-        py = by_ * (64u >> sh) + (lane >> sh);
-    }
-    f3 o, d;
-    if (!p.gen_px(px, py, o, d)) return;
-    RadianceTraceResult r = trace_radiance<S, kCount>(rt, fp, o, d, has_prev, stack);
-    p.finish_px(px, py, o, d, r);
-}
-
-template <class S, bool kCount>
-__device__ __forceinline__ void k_diff_sample_gen_body(const FrameParams& fp, const TraceRes& rt, const vgi_ind_diff_sample_gen_io& io, const vgi_pc_sample_gen& pc, uint32_t bx_, uint32_t by_) {
-    const DiffGenPass<S> p{fp, io, pc};
-    sample_pixel<DiffGenPass<S>, S, kCount>(p, rt, fp, pc.has_prev_frame != 0, bx_, by_);
-}
-
-template <class S, bool kCount>
-__global__ void __launch_bounds__(64, kTraceWaves) k_diff_sample_gen(FrameParams fp, TraceRes rt, vgi_ind_diff_sample_gen_io io, vgi_pc_sample_gen pc) {
-    k_diff_sample_gen_body<S, kCount>(fp, rt, io, pc, blockIdx.x, blockIdx.y);
-}
 
 template <class S>
 struct DiffValidatePass {
@@ -135,17 +103,6 @@ struct DiffValidatePass {
         S::st3(io.rw_hit_radiance_texture, i, r.radiance);
     }
 };
-
-template <class S, bool kCount>
-__device__ __forceinline__ void k_diff_sample_validate_body(const FrameParams& fp, const TraceRes& rt, const vgi_ind_diff_sample_validate_io& io, uint32_t bx_, uint32_t by_) {
-    const DiffValidatePass<S> p{fp, io};
-    sample_pixel<DiffValidatePass<S>, S, kCount>(p, rt, fp, true, bx_, by_);
-}
-
-template <class S, bool kCount>
-__global__ void __launch_bounds__(64, kTraceWaves) k_diff_sample_validate(FrameParams fp, TraceRes rt, vgi_ind_diff_sample_validate_io io) {
-    k_diff_sample_validate_body<S, kCount>(fp, rt, io, blockIdx.x, blockIdx.y);
-}
 
 // GGX VNDF sample [Heitz 2014] of ind_spec_sample_gen.hlsl:67-120; returns the
 // reflected world-space direction.
@@ -219,17 +176,6 @@ struct SpecGenPass {
     }
 };
 
-template <class S, bool kCount>
-__device__ __forceinline__ void k_spec_sample_gen_body(const FrameParams& fp, const TraceRes& rt, const vgi_ind_spec_sample_gen_io& io, const vgi_pc_sample_gen& pc, uint32_t bx_, uint32_t by_) {
-    const SpecGenPass<S> p{fp, io, pc};
-    sample_pixel<SpecGenPass<S>, S, kCount>(p, rt, fp, pc.has_prev_frame != 0, bx_, by_);
-}
-
-template <class S, bool kCount>
-__global__ void __launch_bounds__(64, kTraceWaves) k_spec_sample_gen(FrameParams fp, TraceRes rt, vgi_ind_spec_sample_gen_io io, vgi_pc_sample_gen pc) {
-    k_spec_sample_gen_body<S, kCount>(fp, rt, io, pc, blockIdx.x, blockIdx.y);
-}
-
 template <class S>
 struct SpecValidatePass {
     const FrameParams& fp;
@@ -269,16 +215,76 @@ struct SpecValidatePass {
     }
 };
 
-template <class S, bool kCount>
-__device__ __forceinline__ void k_spec_sample_validate_body(const FrameParams& fp, const TraceRes& rt, const vgi_ind_spec_sample_validate_io& io, uint32_t bx_, uint32_t by_) {
-    const SpecValidatePass<S> p{fp, rt, io};
-    sample_pixel<SpecValidatePass<S>, S, kCount>(p, rt, fp, true, bx_, by_);
+// One pass's lane per pixel of tile (bx_, by_): 8x8 pixels in 2x2 quads, or
+// rows of rt.tile_w pixels (16 x 4, 32 x 2); the shape is a launch parameter
+// (vgi_tuning) and does not change any pixel's result.
+template <class P, class S, bool kCount>
+__device__ __forceinline__ void sample_pixel(const P& p, const TraceRes& rt, const FrameParams& fp, bool has_prev,
+                                             uint32_t bx_, uint32_t by_) {
+    VGI_TRAVERSAL_STACK(stack);
+    uint32_t px, py;
+    if (rt.tile_w == 8u) {
+        quad_tile_pixel_at<8>(bx_, by_, px, py);
+    } else {
+        const uint32_t lane = threadIdx.x & 63u, sh = rt.tile_w == 16u ? 4u : 5u;
+        px = (bx_ << sh) + (lane & (rt.tile_w - 1u));
+        py = by_ * (64u >> sh) + (lane >> sh);
+    }
+    f3 o, d;
+    if (!p.gen_px(px, py, o, d)) return;
+    RadianceTraceResult r = trace_radiance<S, kCount>(rt, fp, o, d, has_prev, stack);
+    p.finish_px(px, py, o, d, r);
 }
 
-template <class S, bool kCount>
-__global__ void __launch_bounds__(64, kTraceWaves) k_spec_sample_validate(FrameParams fp, TraceRes rt, vgi_ind_spec_sample_validate_io io) {
-    k_spec_sample_validate_body<S, kCount>(fp, rt, io, blockIdx.x, blockIdx.y);
+// One lobe's generation and validation as one pass: the two differ in the
+// code that makes a pixel's ray and that writes its sample, and share the
+// traversals and the shading between them.  `validate` is the same for the
+// whole wave.
+template <class Gen, class Val>
+struct LobePass {
+    bool validate;
+    Gen gen;
+    Val val;
+    __device__ bool gen_px(uint32_t px, uint32_t py, f3& o, f3& d) const {
+        return validate ? val.gen_px(px, py, o, d) : gen.gen_px(px, py, o, d);
+    }
+    __device__ void finish_px(uint32_t px, uint32_t py, f3 o, f3 d, const RadianceTraceResult& r) const {
+        if (validate)
+            val.finish_px(px, py, o, d, r);
+        else
+            gen.finish_px(px, py, o, d, r);
+    }
+};
+
+template <class S, bool kSpec, bool kCount>
+__device__ __forceinline__ void k_sample_rays_body(const FrameParams& fp, const TraceRes& rt, const SampleSet& a,
+                                                   uint32_t pass, uint32_t bx_, uint32_t by_) {
+    if constexpr (kSpec) {
+        const bool v = pass == kSampleSpecValidate;
+        const LobePass<SpecGenPass<S>, SpecValidatePass<S>> p{v, {fp, a.spec_gen, a.spec_pc}, {fp, rt, a.spec_validate}};
+        sample_pixel<decltype(p), S, kCount>(p, rt, fp, v || a.spec_pc.has_prev_frame != 0, bx_, by_);
+    } else {
+        const bool v = pass == kSampleDiffValidate;
+        const LobePass<DiffGenPass<S>, DiffValidatePass<S>> p{v, {fp, a.diff_gen, a.diff_pc}, {fp, a.diff_validate}};
+        sample_pixel<decltype(p), S, kCount>(p, rt, fp, v || a.diff_pc.has_prev_frame != 0, bx_, by_);
+    }
 }
+
+// The ray passes of a view's frame and lobe in one launch, part blockIdx.z =
+// one pass.  A ray pass's last waves (its longest rays, about 100 us of serial
+// node visits) run on a nearly empty chip; with the specular validation in
+// the generation's launch instead of ahead of the diffuse generation a frame
+// has one such end less: 256x256 frame 474 -> 384 us, 803x451 577 -> 531 us,
+// 1080p 1628 -> 1597 us, four small views in a batch 991 -> 918 us; 16 views
+// of 14 Mpix in all stay at 11.4 ms.
+template <class S, bool kSpec, bool kCount>
+__global__ void __launch_bounds__(64, kTraceWaves) k_sample_rays(FrameParams fp, TraceRes rt, SampleSet a) {
+    k_sample_rays_body<S, kSpec, kCount>(fp, rt, a, a.pass[blockIdx.z], blockIdx.x, blockIdx.y);
+}
+template <class S, bool kCount>
+constexpr auto k_sample_spec_rays = k_sample_rays<S, true, kCount>;
+template <class S, bool kCount>
+constexpr auto k_sample_diff_rays = k_sample_rays<S, false, kCount>;
 
 // One cache ray: hash_grid_raygen.hlsl:141-204 for compacted query `id`.
 // With `staging` the blended radiance goes to staging[id] (4 floats) and
@@ -408,42 +414,14 @@ static FrameParams to_fp(const vgi_frame_params* fp) {
 // Fused multi-view launches (vgi_batch.h); the scene (and so the LDS stack
 // size) is shared by every view of a batch.
 // ---------------------------------------------------------------------------
-template <class S>
-struct JobDiffGen {
+template <class S, bool kSpec>
+struct JobSampleRays {
     FrameParams fp;
     TraceRes rt;
-    vgi_ind_diff_sample_gen_io io;
-    vgi_pc_sample_gen pc;
-    __device__ static void run(const JobDiffGen& j, uint32_t bx, uint32_t by) {
-        k_diff_sample_gen_body<S, false>(j.fp, j.rt, j.io, j.pc, bx, by);
-    }
-};
-template <class S>
-struct JobDiffValidate {
-    FrameParams fp;
-    TraceRes rt;
-    vgi_ind_diff_sample_validate_io io;
-    __device__ static void run(const JobDiffValidate& j, uint32_t bx, uint32_t by) {
-        k_diff_sample_validate_body<S, false>(j.fp, j.rt, j.io, bx, by);
-    }
-};
-template <class S>
-struct JobSpecGen {
-    FrameParams fp;
-    TraceRes rt;
-    vgi_ind_spec_sample_gen_io io;
-    vgi_pc_sample_gen pc;
-    __device__ static void run(const JobSpecGen& j, uint32_t bx, uint32_t by) {
-        k_spec_sample_gen_body<S, false>(j.fp, j.rt, j.io, j.pc, bx, by);
-    }
-};
-template <class S>
-struct JobSpecValidate {
-    FrameParams fp;
-    TraceRes rt;
-    vgi_ind_spec_sample_validate_io io;
-    __device__ static void run(const JobSpecValidate& j, uint32_t bx, uint32_t by) {
-        k_spec_sample_validate_body<S, false>(j.fp, j.rt, j.io, bx, by);
+    SampleSet a;
+    uint32_t tiles_y;  // tile rows of one pass: a view's tile grid holds its passes one below the other
+    __device__ static void run(const JobSampleRays& j, uint32_t bx, uint32_t by) {
+        k_sample_rays_body<S, kSpec, false>(j.fp, j.rt, j.a, j.a.pass[by / j.tiles_y], bx, by % j.tiles_y);
     }
 };
 struct HgRaygenArgs {
@@ -466,85 +444,82 @@ struct JobHgOApply : HgRaygenArgs {
 static_assert(sizeof(JobHgOApply<StorageF32>) == sizeof(JobHgRaygen<StorageF32>), "one table, two launches");
 static_assert(kRaygenGroups * 64 >= kHashGridMaxQueries, "the cache-ray tiles cover the compact list");
 template <class S>
-struct BatchMinWaves<JobDiffGen<S>> {
+struct JobDiffRays : JobSampleRays<S, false> {};
+template <class S>
+struct JobSpecRays : JobSampleRays<S, true> {};
+static_assert(sizeof(JobDiffRays<StorageF32>) == sizeof(JobSpecRays<StorageF32>), "one table, two launches");
+template <class S>
+struct BatchMinWaves<JobDiffRays<S>> {
     static constexpr int value = kTraceWaves;
 };
 template <class S>
-struct BatchMinWaves<JobDiffValidate<S>> {
-    static constexpr int value = kTraceWaves;
-};
-template <class S>
-struct BatchMinWaves<JobSpecGen<S>> {
-    static constexpr int value = kTraceWaves;
-};
-template <class S>
-struct BatchMinWaves<JobSpecValidate<S>> {
+struct BatchMinWaves<JobSpecRays<S>> {
     static constexpr int value = kTraceWaves;
 };
 
-static vgi_status fill_diff_gen(const PassRec* const* recs, int n, void* host) {
-    auto* t = batch_table<JobDiffGen>(host);
-    for (int v = 0; v < n; ++v) {
-        const PassRec& r = *recs[v];
-        auto& j = t->jobs[v];
-        vgi_status s = make_trace_res(&r.tr, r.pc.sample_gen.has_prev_frame != 0, j.rt);
-        if (s != VGI_OK) return s;
-        j.fp = to_fp(&r.fp);
-        j.io = r.io.diff_gen;
-        j.pc = r.pc.sample_gen;
-        {
-            const dim3 tg = trace_tile_grid(j.io.width, j.io.height, j.rt.tile_w);
-            batch_add_tiles(t->hd, v, tg.x, tg.y);
+// What the entry points of the single passes check, for each pass of a set;
+// its trace resources and its image size.
+static vgi_status check_sample_set(const vgi_trace_resources* tr, const SampleSet& a, TraceRes& t, uint32_t& w,
+                                   uint32_t& h) {
+    bool need_prev = false;
+    w = h = 0;
+    for (uint32_t k = 0; k < a.count; ++k) {
+        uint32_t pw, ph, storage;
+        bool bound;
+        switch (a.pass[k]) {
+            case kSampleSpecValidate: {
+                const auto& io = a.spec_validate;
+                pw = io.width, ph = io.height, storage = io.storage;
+                bound = io.rw_prev_reservoir_texture && io.rw_prev_hit_pos_texture && io.rw_prev_hit_radiance_texture;
+                need_prev = true;
+                break;
+            }
+            case kSampleDiffGen: {
+                const auto& io = a.diff_gen;
+                pw = io.width, ph = io.height, storage = io.storage;
+                bound = io.gbuffer_color && io.gbuffer_depth && io.rw_hit_pos_normal_texture && io.rw_hit_radiance_texture;
+                need_prev |= a.diff_pc.has_prev_frame != 0;
+                break;
+            }
+            case kSampleDiffValidate: {
+                const auto& io = a.diff_validate;
+                pw = io.width, ph = io.height, storage = io.storage;
+                bound = io.depth_texture && io.rw_reservoir_texture && io.rw_hit_pos_normal_texture &&
+                        io.rw_hit_radiance_texture;
+                need_prev = true;
+                break;
+            }
+            default: {
+                const auto& io = a.spec_gen;
+                pw = io.width, ph = io.height, storage = io.storage;
+                bound = io.gbuffer_color && io.gbuffer_depth && io.rw_hit_pos_texture && io.rw_hit_radiance_texture;
+                need_prev |= a.spec_pc.has_prev_frame != 0;
+                break;
+            }
         }
+        VGI_REQUIRE(valid_dims(pw, ph), "sample rays: bad size");
+        VGI_REQUIRE(tr && storage == tr->storage, "sample rays: storage mismatch");
+        VGI_REQUIRE(bound, "sample rays: missing binding");
+        VGI_REQUIRE(k == 0 || (pw == w && ph == h), "internal: sample passes of different sizes");
+        w = pw;
+        h = ph;
     }
-    return VGI_OK;
+    VGI_REQUIRE(a.count > 0, "internal: no sample pass");
+    return make_trace_res(tr, need_prev, t);
 }
-static vgi_status fill_diff_validate(const PassRec* const* recs, int n, void* host) {
-    auto* t = batch_table<JobDiffValidate>(host);
+
+static vgi_status fill_sample_rays(const PassRec* const* recs, int n, void* host) {
+    auto* t = batch_table<JobDiffRays>(host);
     for (int v = 0; v < n; ++v) {
         const PassRec& r = *recs[v];
         auto& j = t->jobs[v];
-        vgi_status s = make_trace_res(&r.tr, true, j.rt);
-        if (s != VGI_OK) return s;
+        uint32_t w, h;
+        VGI_CHECK(check_sample_set(&r.tr, r.io.sample, j.rt, w, h));
         j.fp = to_fp(&r.fp);
-        j.io = r.io.diff_validate;
-        {
-            const dim3 tg = trace_tile_grid(j.io.width, j.io.height, j.rt.tile_w);
-            batch_add_tiles(t->hd, v, tg.x, tg.y);
-        }
-    }
-    return VGI_OK;
-}
-static vgi_status fill_spec_gen(const PassRec* const* recs, int n, void* host) {
-    auto* t = batch_table<JobSpecGen>(host);
-    for (int v = 0; v < n; ++v) {
-        const PassRec& r = *recs[v];
-        auto& j = t->jobs[v];
-        vgi_status s = make_trace_res(&r.tr, r.pc.sample_gen.has_prev_frame != 0, j.rt);
-        if (s != VGI_OK) return s;
-        j.fp = to_fp(&r.fp);
-        j.io = r.io.spec_gen;
-        j.pc = r.pc.sample_gen;
-        {
-            const dim3 tg = trace_tile_grid(j.io.width, j.io.height, j.rt.tile_w);
-            batch_add_tiles(t->hd, v, tg.x, tg.y);
-        }
-    }
-    return VGI_OK;
-}
-static vgi_status fill_spec_validate(const PassRec* const* recs, int n, void* host) {
-    auto* t = batch_table<JobSpecValidate>(host);
-    for (int v = 0; v < n; ++v) {
-        const PassRec& r = *recs[v];
-        auto& j = t->jobs[v];
-        vgi_status s = make_trace_res(&r.tr, true, j.rt);
-        if (s != VGI_OK) return s;
-        j.fp = to_fp(&r.fp);
-        j.io = r.io.spec_validate;
-        {
-            const dim3 tg = trace_tile_grid(j.io.width, j.io.height, j.rt.tile_w);
-            batch_add_tiles(t->hd, v, tg.x, tg.y);
-        }
+        j.a = r.io.sample;
+        const dim3 tg = trace_tile_grid(w, h, j.rt.tile_w);
+        j.tiles_y = tg.y;
+        batch_add_tiles(t->hd, v, tg.x, tg.y * j.a.count);
     }
     return VGI_OK;
 }
@@ -587,23 +562,17 @@ static vgi_status launch_hg_oraygen(const void* dev, uint32_t storage, uint32_t 
 }
 
 const BatchOps* batch_ops_sample(int kind) {
-    static const BatchOps diff_gen{sizeof(BatchTable<JobDiffGen<StorageF32>>), fill_diff_gen, batch_launch<JobDiffGen>,
-                                   64, true};
-    static const BatchOps diff_validate{sizeof(BatchTable<JobDiffValidate<StorageF32>>), fill_diff_validate,
-                                        batch_launch<JobDiffValidate>, 64, true};
-    static const BatchOps spec_gen{sizeof(BatchTable<JobSpecGen<StorageF32>>), fill_spec_gen, batch_launch<JobSpecGen>,
-                                   64, true};
-    static const BatchOps spec_validate{sizeof(BatchTable<JobSpecValidate<StorageF32>>), fill_spec_validate,
-                                        batch_launch<JobSpecValidate>, 64, true};
+    static const BatchOps spec_rays{sizeof(BatchTable<JobSpecRays<StorageF32>>), fill_sample_rays,
+                                    batch_launch<JobSpecRays>, 64, true};
+    static const BatchOps diff_rays{sizeof(BatchTable<JobDiffRays<StorageF32>>), fill_sample_rays,
+                                    batch_launch<JobDiffRays>, 64, true};
     static const BatchOps hg_raygen{sizeof(BatchTable<JobHgRaygen<StorageF32>>), fill_hg_raygen,
                                     batch_launch<JobHgRaygen>, 64, true};
     static const BatchOps hg_oraygen{sizeof(BatchTable<JobHgRaygen<StorageF32>>), fill_hg_oraygen, launch_hg_oraygen,
                                      64, true};
     switch (kind) {
-        case kPassDiffGen: return &diff_gen;
-        case kPassDiffValidate: return &diff_validate;
-        case kPassSpecGen: return &spec_gen;
-        case kPassSpecValidate: return &spec_validate;
+        case kPassSampleSpec: return &spec_rays;
+        case kPassSampleDiff: return &diff_rays;
         case kPassHgRaygen: return &hg_raygen;
         case kPassHgRaygenOrdered: return &hg_oraygen;
         default: return nullptr;
@@ -614,77 +583,78 @@ const BatchOps* batch_ops_sample(int kind) {
 
 using namespace vgi;
 
-extern "C" vgi_status vgi_pass_ind_diff_sample_gen(const vgi_frame_params* fp, const vgi_trace_resources* rt,
-                                                   const vgi_ind_diff_sample_gen_io* io, const vgi_pc_sample_gen* pc,
-                                                   void* stream) {
-    VGI_REQUIRE(fp && io && pc, "vgi_pass_ind_diff_sample_gen: null argument");
-    VGI_REQUIRE(valid_dims(io->width, io->height), "vgi_pass_ind_diff_sample_gen: bad size");
-    VGI_REQUIRE(io->storage == rt->storage, "vgi_pass_ind_diff_sample_gen: storage mismatch");
-    VGI_REQUIRE(io->gbuffer_color && io->gbuffer_depth && io->rw_hit_pos_normal_texture && io->rw_hit_radiance_texture,
-                "vgi_pass_ind_diff_sample_gen: missing binding");
+// One launch of the set's passes (`name` and `bytes`: its entry in the profiler).
+static vgi_status launch_sample_set(const char* name, double bytes, const vgi_frame_params* fp,
+                                    const vgi_trace_resources* tr, const SampleSet& a, hipStream_t st) {
     TraceRes t;
-    vgi_status s = make_trace_res(rt, pc->has_prev_frame != 0, t);
-    if (s != VGI_OK) return s;
-    hipStream_t st = (hipStream_t)stream;
-    ProfScope prof("ind_diff_sample_gen", st, (double)io->width * io->height * (8 + 4 + 8 + radiance_bytes(io->storage)));
-    VGI_DISPATCH_STORAGE(io->storage, k_diff_sample_gen, trace_tile_grid(io->width, io->height, t.tile_w), to_fp(fp), t, *io, *pc);
-    trace_stats_collect("ind_diff_sample_gen", st);
-    return check_launch("k_diff_sample_gen");
+    uint32_t w, h;
+    VGI_CHECK(check_sample_set(tr, a, t, w, h));
+    ProfScope prof(name, st, (double)w * h * bytes);
+    dim3 g = trace_tile_grid(w, h, t.tile_w);
+    g.z = a.count;
+    if (a.spec())
+        VGI_DISPATCH_STORAGE(tr->storage, k_sample_spec_rays, g, to_fp(fp), t, a);
+    else
+        VGI_DISPATCH_STORAGE(tr->storage, k_sample_diff_rays, g, to_fp(fp), t, a);
+    trace_stats_collect(name, st);
+    return check_launch("k_sample_rays");
+}
+
+namespace vgi {
+// The renderer's sample passes.  Under the per-pass timers and the traversal
+// statistics each runs as its own launch, so that it has its own figures.
+vgi_status launch_sample_rays(const PassRec& r, hipStream_t st) {
+    const SampleSet& a = r.io.sample;
+    void* s = (void*)st;
+    if (!trace_counters() && !profiling_pass("ind_diff_sample_gen") && !profiling_pass("ind_diff_sample_validate") &&
+        !profiling_pass("ind_spec_sample_gen") && !profiling_pass("ind_spec_sample_validate"))
+        return launch_sample_set(a.spec() ? "ind_spec_sample" : "ind_diff_sample", 0.0, &r.fp, &r.tr, a, st);
+    for (uint32_t k = 0; k < a.count; ++k) switch (a.pass[k]) {
+            case kSampleSpecValidate: VGI_CHECK(vgi_pass_ind_spec_sample_validate(&r.fp, &r.tr, &a.spec_validate, s)); break;
+            case kSampleDiffGen: VGI_CHECK(vgi_pass_ind_diff_sample_gen(&r.fp, &r.tr, &a.diff_gen, &a.diff_pc, s)); break;
+            case kSampleDiffValidate: VGI_CHECK(vgi_pass_ind_diff_sample_validate(&r.fp, &r.tr, &a.diff_validate, s)); break;
+            default: VGI_CHECK(vgi_pass_ind_spec_sample_gen(&r.fp, &r.tr, &a.spec_gen, &a.spec_pc, s)); break;
+        }
+    return VGI_OK;
+}
+}  // namespace vgi
+
+extern "C" vgi_status vgi_pass_ind_diff_sample_gen(const vgi_frame_params* fp, const vgi_trace_resources* rt,
+                                                   const vgi_ind_diff_sample_gen_io* io, const vgi_pc_sample_gen* pc, void* stream) {
+    VGI_REQUIRE(fp && rt && io && pc, "vgi_pass_ind_diff_sample_gen: null argument");
+    SampleSet a{};
+    a.diff_gen = *io;
+    a.diff_pc = *pc;
+    a.add(kSampleDiffGen);
+    return launch_sample_set("ind_diff_sample_gen", (double)(8 + 4 + 8 + radiance_bytes(io->storage)), fp, rt, a, (hipStream_t)stream);
 }
 
 extern "C" vgi_status vgi_pass_ind_diff_sample_validate(const vgi_frame_params* fp, const vgi_trace_resources* rt,
                                                         const vgi_ind_diff_sample_validate_io* io, void* stream) {
-    VGI_REQUIRE(fp && io, "vgi_pass_ind_diff_sample_validate: null argument");
-    VGI_REQUIRE(valid_dims(io->width, io->height), "vgi_pass_ind_diff_sample_validate: bad size");
-    VGI_REQUIRE(io->storage == rt->storage, "vgi_pass_ind_diff_sample_validate: storage mismatch");
-    VGI_REQUIRE(io->depth_texture && io->rw_reservoir_texture && io->rw_hit_pos_normal_texture &&
-                    io->rw_hit_radiance_texture,
-                "vgi_pass_ind_diff_sample_validate: missing binding");
-    TraceRes t;
-    vgi_status s = make_trace_res(rt, true, t);
-    if (s != VGI_OK) return s;
-    hipStream_t st = (hipStream_t)stream;
-    ProfScope prof("ind_diff_sample_validate", st,
-                   (double)io->width * io->height * (4 + 2 * (4 + 8 + radiance_bytes(io->storage))));
-    VGI_DISPATCH_STORAGE(io->storage, k_diff_sample_validate, trace_tile_grid(io->width, io->height, t.tile_w), to_fp(fp), t, *io);
-    trace_stats_collect("ind_diff_sample_validate", st);
-    return check_launch("k_diff_sample_validate");
+    VGI_REQUIRE(fp && rt && io, "vgi_pass_ind_diff_sample_validate: null argument");
+    SampleSet a{};
+    a.diff_validate = *io;
+    a.add(kSampleDiffValidate);
+    return launch_sample_set("ind_diff_sample_validate", (double)(4 + 2 * (4 + 8 + radiance_bytes(io->storage))), fp, rt, a, (hipStream_t)stream);
 }
 
 extern "C" vgi_status vgi_pass_ind_spec_sample_gen(const vgi_frame_params* fp, const vgi_trace_resources* rt,
-                                                   const vgi_ind_spec_sample_gen_io* io, const vgi_pc_sample_gen* pc,
-                                                   void* stream) {
-    VGI_REQUIRE(fp && io && pc, "vgi_pass_ind_spec_sample_gen: null argument");
-    VGI_REQUIRE(valid_dims(io->width, io->height), "vgi_pass_ind_spec_sample_gen: bad size");
-    VGI_REQUIRE(io->storage == rt->storage, "vgi_pass_ind_spec_sample_gen: storage mismatch");
-    VGI_REQUIRE(io->gbuffer_color && io->gbuffer_depth && io->rw_hit_pos_texture && io->rw_hit_radiance_texture,
-                "vgi_pass_ind_spec_sample_gen: missing binding");
-    TraceRes t;
-    vgi_status s = make_trace_res(rt, pc->has_prev_frame != 0, t);
-    if (s != VGI_OK) return s;
-    hipStream_t st = (hipStream_t)stream;
-    ProfScope prof("ind_spec_sample_gen", st, (double)io->width * io->height * (4 + 4 + 16 + radiance_bytes(io->storage)));
-    VGI_DISPATCH_STORAGE(io->storage, k_spec_sample_gen, trace_tile_grid(io->width, io->height, t.tile_w), to_fp(fp), t, *io, *pc);
-    trace_stats_collect("ind_spec_sample_gen", st);
-    return check_launch("k_spec_sample_gen");
+                                                   const vgi_ind_spec_sample_gen_io* io, const vgi_pc_sample_gen* pc, void* stream) {
+    VGI_REQUIRE(fp && rt && io && pc, "vgi_pass_ind_spec_sample_gen: null argument");
+    SampleSet a{};
+    a.spec_gen = *io;
+    a.spec_pc = *pc;
+    a.add(kSampleSpecGen);
+    return launch_sample_set("ind_spec_sample_gen", (double)(4 + 4 + 16 + radiance_bytes(io->storage)), fp, rt, a, (hipStream_t)stream);
 }
 
 extern "C" vgi_status vgi_pass_ind_spec_sample_validate(const vgi_frame_params* fp, const vgi_trace_resources* rt,
                                                         const vgi_ind_spec_sample_validate_io* io, void* stream) {
-    VGI_REQUIRE(fp && io, "vgi_pass_ind_spec_sample_validate: null argument");
-    VGI_REQUIRE(valid_dims(io->width, io->height), "vgi_pass_ind_spec_sample_validate: bad size");
-    VGI_REQUIRE(io->storage == rt->storage, "vgi_pass_ind_spec_sample_validate: storage mismatch");
-    VGI_REQUIRE(io->rw_prev_reservoir_texture && io->rw_prev_hit_pos_texture && io->rw_prev_hit_radiance_texture,
-                "vgi_pass_ind_spec_sample_validate: missing binding");
-    TraceRes t;
-    vgi_status s = make_trace_res(rt, true, t);
-    if (s != VGI_OK) return s;
-    hipStream_t st = (hipStream_t)stream;
-    ProfScope prof("ind_spec_sample_validate", st,
-                   (double)io->width * io->height * (4 + 2 * (8 + 16 + radiance_bytes(io->storage))));
-    VGI_DISPATCH_STORAGE(io->storage, k_spec_sample_validate, trace_tile_grid(io->width, io->height, t.tile_w), to_fp(fp), t, *io);
-    trace_stats_collect("ind_spec_sample_validate", st);
-    return check_launch("k_spec_sample_validate");
+    VGI_REQUIRE(fp && rt && io, "vgi_pass_ind_spec_sample_validate: null argument");
+    SampleSet a{};
+    a.spec_validate = *io;
+    a.add(kSampleSpecValidate);
+    return launch_sample_set("ind_spec_sample_validate", (double)(4 + 2 * (8 + 16 + radiance_bytes(io->storage))), fp, rt, a, (hipStream_t)stream);
 }
 
 extern "C" vgi_status vgi_pass_hash_grid_raygen(const vgi_frame_params* fp, const vgi_trace_resources* rt,

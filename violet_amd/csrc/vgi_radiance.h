@@ -283,14 +283,20 @@ __device__ __forceinline__ RadianceTraceResult radiance_at(const TraceRes& rt, c
 }
 
 // raytrace.inc.hlsl:65-208: closest hit of (o, d), then the sun shadow ray
-// from the hit (any hit), then radiance_at.
+// from the hit (any hit) where the sun can reach it, then radiance_at.
 template <class S, bool kCount = false>
 __device__ __forceinline__ RadianceTraceResult trace_radiance(const TraceRes& rt, const FrameParams& fp, f3 o, f3 d,
                                                               bool has_prev_frame, LdsStack stack) {
     Hit hit = trace_closest<kCount>(rt.scene, o, d, kRayTMin, kRayTMax, stack);
     SurfaceHit sh = shade_hit(rt.scene, hit, d);
+    // A surface that faces away from the sun gets no light from it whether or
+    // not something is in between (a finite BRDF and sun times a cosine of
+    // zero): no ray.  1080p frame 1591 -> 1577 us.
     bool sun_visible = false;
-    if (!sh.missed) sun_visible = !trace_any<kCount>(rt.scene, sh.position, xyz(fp.sun_dir), kRayTMin, kRayTMax, stack);
+    const f3 si = xyz(fp.sun_inten);
+    const bool away = !(dot3(sh.normal, xyz(fp.sun_dir)) > 0.0f) && fabsf(si.x) + fabsf(si.y) + fabsf(si.z) < INFINITY;
+    if (!sh.missed && !away)
+        sun_visible = !trace_any<kCount>(rt.scene, sh.position, xyz(fp.sun_dir), kRayTMin, kRayTMax, stack);
     return radiance_at<S>(rt, fp, o, d, sh, sun_visible, has_prev_frame);
 }
 

@@ -323,7 +323,8 @@ __device__ __forceinline__ void k_hgo_claim_body(const HashQuery* queries, const
 }
 
 // Compaction in cell order: `count` stores each wave's number of selected
-// cells (and, wave 0, the counter's value on entry) in the workspace;
+// cells (and, wave 0, the counter's value on entry, or 0 without a counter) in
+// the workspace;
 // `place` sums the counts of the waves before it and writes its cells there.
 // Selected words have bit 31 set.
 __device__ __forceinline__ uint64_t compact_lane_mask(const uint32_t* selection, uint32_t first) {
@@ -351,13 +352,13 @@ __device__ __forceinline__ void k_hgo_count_body(const uint32_t* selection, cons
     const uint32_t total = wave_sum((uint32_t)__popcll(act));
     if (lane == 0) {
         G(ws)[bx_] = total;
-        if (bx_ == 0) G(ws)[kCompactWaves] = G(counter)[0];
+        if (bx_ == 0) G(ws)[kCompactWaves] = counter ? G(counter)[0] : 0u;
     }
 }
 
 __device__ __forceinline__ void k_hgo_place_body(uint32_t* selection, uint32_t* winner,
                                                  uint32_t* out_index, uint32_t* out_addr, uint32_t* out_counter,
-                                                 const uint32_t* ws, uint32_t bx_) {
+                                                 uint32_t* clear_word, const uint32_t* ws, uint32_t bx_) {
     static_assert(kCompactWaves == 4 * 64, "four wave counts per lane");
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t before = 0, all = 0;
@@ -370,7 +371,10 @@ __device__ __forceinline__ void k_hgo_place_body(uint32_t* selection, uint32_t* 
     before = wave_sum(before);
     all = wave_sum(all);
     const uint32_t start = G(ws)[kCompactWaves];
-    if (bx_ == kCompactWaves - 1 && lane == 0) G(out_counter)[0] = start + all;
+    if (bx_ == kCompactWaves - 1 && lane == 0) {
+        G(out_counter)[0] = start + all;
+        if (clear_word) G(clear_word)[0] = 0u;
+    }
     const uint32_t first = bx_ * kCompactCellsPerWave + lane * kCompactCellsPerLane;
     uint64_t act = compact_lane_mask(selection, first);
     const uint32_t cnt = (uint32_t)__popcll(act);
@@ -418,8 +422,8 @@ __global__ void __launch_bounds__(64) k_hgo_count(const uint32_t* selection, con
 }
 __global__ void __launch_bounds__(64) k_hgo_place(uint32_t* selection, uint32_t* winner,
                                                   uint32_t* out_index, uint32_t* out_addr, uint32_t* out_counter,
-                                                  const uint32_t* ws) {
-    k_hgo_place_body(selection, winner, out_index, out_addr, out_counter, ws, blockIdx.x);
+                                                  uint32_t* clear_word, const uint32_t* ws) {
+    k_hgo_place_body(selection, winner, out_index, out_addr, out_counter, clear_word, ws, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -488,18 +492,19 @@ struct JobHgOClaim : HgOSelectArgs {
 };
 struct HgOCompactArgs {
     uint32_t *selection, *winner;
-    uint32_t *out_index, *out_addr, *out_counter, *ws;
+    uint32_t *out_index, *out_addr, *out_counter, *ws, *clear_word;
+    const uint32_t* start;  // the counter's value on entry (null: zero)
 };
 template <class>
 struct JobHgOCount : HgOCompactArgs {
     __device__ static void run(const JobHgOCount& j, uint32_t bx, uint32_t) {
-        k_hgo_count_body(j.selection, j.out_counter, j.ws, bx);
+        k_hgo_count_body(j.selection, j.start, j.ws, bx);
     }
 };
 template <class>
 struct JobHgOPlace : HgOCompactArgs {
     __device__ static void run(const JobHgOPlace& j, uint32_t bx, uint32_t) {
-        k_hgo_place_body(j.selection, j.winner, j.out_index, j.out_addr, j.out_counter, j.ws, bx);
+        k_hgo_place_body(j.selection, j.winner, j.out_index, j.out_addr, j.out_counter, j.clear_word, j.ws, bx);
     }
 };
 static_assert(sizeof(JobHgOGather<StorageF32>) == sizeof(HgOSelectArgs) &&
@@ -579,6 +584,8 @@ static vgi_status fill_hg_ocompact(const PassRec* const* recs, int n, void* host
         a.out_addr = io.rw_compact_query_cell_addr_buffer;
         a.out_counter = io.rw_compact_query_counter_buffer;
         a.ws = io.rw_workspace_buffer;
+        a.clear_word = (uint32_t*)recs[v]->clear_ptr;
+        a.start = nullptr;
         batch_add_tiles(t->hd, v, kCompactWaves, 1);
     }
     return VGI_OK;
@@ -680,8 +687,9 @@ extern "C" vgi_status vgi_pass_hash_grid_query_select_ordered(const vgi_hash_gri
     return check_launch("k_hgo_claim");
 }
 
-extern "C" vgi_status vgi_pass_hash_grid_query_compact_ordered(const vgi_hash_grid_ordered_compact_io* io,
-                                                               void* stream) {
+// The compaction; `counter`: where its count starts from (null: zero), `clear_word` (may be null): set to zero by it.
+static vgi_status launch_compact_ordered(const vgi_hash_grid_ordered_compact_io* io, const uint32_t* counter,
+                                         uint32_t* clear_word, hipStream_t st) {
     VGI_REQUIRE(io && io->rw_hash_grid_query_selection_buffer && io->rw_hash_grid_query_winner_buffer &&
                     io->rw_compact_query_index_buffer && io->rw_compact_query_cell_addr_buffer &&
                     io->rw_compact_query_counter_buffer && io->rw_workspace_buffer,
@@ -689,17 +697,28 @@ extern "C" vgi_status vgi_pass_hash_grid_query_compact_ordered(const vgi_hash_gr
     VGI_REQUIRE(((uintptr_t)io->rw_hash_grid_query_selection_buffer & 15u) == 0,
                 "vgi_pass_hash_grid_query_compact_ordered: selection buffer not 16-byte aligned");
     static_assert(VGI_HASH_GRID_COMPACT_WORKSPACE_WORDS == kCompactWaves + 1, "workspace size");
-    hipStream_t st = (hipStream_t)stream;
     ProfScope prof("hash_grid_query_compact_ordered", st, (double)kHashGridNumCells * 8.0);
     hipLaunchKernelGGL(k_hgo_count, dim3(kCompactWaves), dim3(64), 0, st, io->rw_hash_grid_query_selection_buffer,
-                       io->rw_compact_query_counter_buffer, io->rw_workspace_buffer);
+                       counter, io->rw_workspace_buffer);
     VGI_CHECK(check_launch("k_hgo_count"));
     hipLaunchKernelGGL(k_hgo_place, dim3(kCompactWaves), dim3(64), 0, st, io->rw_hash_grid_query_selection_buffer,
                        io->rw_hash_grid_query_winner_buffer, io->rw_compact_query_index_buffer,
-                       io->rw_compact_query_cell_addr_buffer, io->rw_compact_query_counter_buffer,
-                       io->rw_workspace_buffer);
+                       io->rw_compact_query_cell_addr_buffer, io->rw_compact_query_counter_buffer, clear_word,
+                       (const uint32_t*)io->rw_workspace_buffer);
     return check_launch("k_hgo_place");
 }
+
+extern "C" vgi_status vgi_pass_hash_grid_query_compact_ordered(const vgi_hash_grid_ordered_compact_io* io,
+                                                               void* stream) {
+    return launch_compact_ordered(io, io ? io->rw_compact_query_counter_buffer : nullptr, nullptr, (hipStream_t)stream);
+}
+
+namespace vgi {
+vgi_status launch_compact_ordered_fresh(const vgi_hash_grid_ordered_compact_io* io, uint32_t* clear_word,
+                                        hipStream_t st) {
+    return launch_compact_ordered(io, nullptr, clear_word, st);
+}
+}  // namespace vgi
 
 static_assert(kHashGridQueryTarget == VGI_HASH_GRID_QUERY_TARGET, "query target");
 

@@ -54,7 +54,8 @@ vgi_status DirectSink::launch(const PassRec& r, hipStream_t st) {
         case kPassHgRaygen: return vgi_pass_hash_grid_raygen(&r.fp, &r.tr, &r.io.hg_raygen, &r.pc.frame_hash, s);
         case kPassHgSelectOrdered:
             return vgi_pass_hash_grid_query_select_ordered(&r.io.hg_oselect, &r.pc.frame_hash, s);
-        case kPassHgCompactOrdered: return vgi_pass_hash_grid_query_compact_ordered(&r.io.hg_ocompact, s);
+        case kPassHgCompactOrdered:
+            return launch_compact_ordered_fresh(&r.io.hg_ocompact, (uint32_t*)r.clear_ptr, st);
         case kPassHgRaygenOrdered:
             return vgi_pass_hash_grid_raygen_ordered(&r.fp, &r.tr, &r.io.hg_oraygen, &r.pc.frame_hash, s);
         case kPassSampleSpec:

@@ -158,7 +158,7 @@ struct PassRec {
     // from) and the spatial pass reads; NULL for the plain entry points
     DiffTap* diff_taps;
     const uint32_t* diff_taps_gbuffer;
-    void* clear_ptr;     // kPassClear
+    void* clear_ptr;     // kPassClear; kPassHgCompactOrdered: a word that the compaction sets to zero besides
     size_t clear_bytes;  // kPassClear
     uint32_t clear_value;  // kPassClear: the 32-bit word every word of the buffer gets (clear_bytes % 4 == 0 unless 0)
 };
@@ -245,6 +245,12 @@ struct DirectSink : PassSink {
     static vgi_status launch(const PassRec& r, hipStream_t st);
 };
 
+// The ordered compaction of a frame: the compact count starts from zero
+// whatever its buffer holds, and `clear_word` becomes zero, so that neither
+// needs a clear of its own (5 us each on the cache update's chain of short
+// launches, which outlasts the G-buffer beside it).
+vgi_status launch_compact_ordered_fresh(const vgi_hash_grid_ordered_compact_io* io, uint32_t* clear_word,
+                                        hipStream_t st);
 // The launch of a kPassSampleSpec or kPassSampleDiff record (vgi_sample.hip).
 vgi_status launch_sample_rays(const PassRec& r, hipStream_t st);
 

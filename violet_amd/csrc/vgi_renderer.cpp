@@ -324,21 +324,22 @@ vgi_status vgi_renderer_plan(vgi_renderer* r, const vgi_scene* scene, const vgi_
             sel.pc.frame_hash = vgi_pc_frame_hash{select_hash};
             CALL(sink.submit(kSlotHgSelect, sel));
         }
-        CALL(sink.submit(kSlotClearCompactCount, make_clear(r->hg_ccount.p, 4)));
+        const int nq = 1 - r->q;
         if (ordered) {
             PassRec cmp = make_rec(kPassHgCompactOrdered);
+            cmp.clear_ptr = r->hg_counter[nq].p;
             cmp.io.hg_ocompact = vgi_hash_grid_ordered_compact_io{
                 r->hg_selection.as<uint32_t>(), r->hg_winner.as<uint32_t>(), r->hg_cidx.as<uint32_t>(),
                 r->hg_caddr.as<uint32_t>(),     r->hg_ccount.as<uint32_t>(), r->hg_workspace.as<uint32_t>()};
             CALL(sink.submit(kSlotHgCompactOrdered, cmp));
         } else {
+            CALL(sink.submit(kSlotClearCompactCount, make_clear(r->hg_ccount.p, 4)));
             PassRec cmp = make_rec(kPassHgCompact);
             cmp.io.hg_compact = vgi_hash_grid_query_compact_io{r->hg_selection.as<uint32_t>(), r->hg_cidx.as<uint32_t>(),
                                                                r->hg_caddr.as<uint32_t>(), r->hg_ccount.as<uint32_t>()};
             CALL(sink.submit(kSlotHgCompact, cmp));
         }
-        const int nq = 1 - r->q;
-        CALL(sink.submit(kSlotClearNextCounter, make_clear(r->hg_counter[nq].p, 4)));
+        if (!ordered) CALL(sink.submit(kSlotClearNextCounter, make_clear(r->hg_counter[nq].p, 4)));
         PassRec rg = make_rec(ordered ? kPassHgRaygenOrdered : kPassHgRaygen, fp);
         rg.tr = trace_res(r, scene, true);
         rg.tr.rw_hash_grid_query_buffer = r->hg_query[nq].as<vgi_hash_grid_query>();

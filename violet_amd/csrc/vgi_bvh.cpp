@@ -618,7 +618,6 @@ extern "C" vgi_status vgi_scene_create(const vgi_scene_desc* desc, vgi_scene** o
     sc->view.num_nodes = (uint32_t)hs.nodes.size();
     sc->view.num_tris = nt;
     sc->view.root = hs.root;
-    sc->view.stack_depth = 3u * sc->depth;  // at most 3 far children pushed per level
     sc->view.counters = nullptr;
     *out = sc;
     return VGI_OK;

@@ -91,7 +91,6 @@ struct SceneView {
     uint32_t num_nodes;
     uint32_t num_tris;
     int32_t root;           // link of the root (node 0)
-    uint32_t stack_depth;   // most traversal-stack entries a ray can hold (3 per node level)
     unsigned long long* counters;  // traversal statistics slots (instrumented kernels only)
 };
 
@@ -110,9 +109,9 @@ constexpr int kSpillEntries = 8;
 constexpr uint32_t kStackMaxEntries = 3 * kBvhMaxDepth;  // 3 far children per 4-wide level
 
 // Register budget of the per-pixel ray-tracing kernels, as waves per SIMD:
-// the traversal hides node-fetch latency with resident waves, and 4 KiB of
-// LDS stack per wave allows more of them than ~80 registers would.  (The
-// cache-ray pass runs too few waves to gain from it and keeps its registers.)
+// 6, 7 and 8 are within 3% of each other (64 registers spill a few values
+// outside the traversal loop; 8 waves hide a node's round trip best).  The
+// cache-ray pass runs too few waves to gain from it and keeps its registers.
 constexpr int kTraceWaves = 8;
 
 // The host side of vgi_scene_create: validation, the binned-SAH build, the
@@ -140,22 +139,5 @@ struct Hit {
     float u, v;  // barycentric weights of vertex 1 and vertex 2
     uint32_t tri;  // scene triangle id; 0xFFFFFFFF = miss
 };
-
-// Moller-Trumbore, two-sided.  Fixed evaluation order (bit-identical on the
-// host and the device).
-VGI_HD bool intersect_tri(f3 o, f3 d, f3 v0, f3 e1, f3 e2, float tmin, float& t, float& u, float& v) {
-    f3 pvec = cross3(d, e2);
-    float det = dot3(e1, pvec);
-    if (det == 0.0f) return false;
-    float inv_det = 1.0f / det;
-    f3 tvec = o - v0;
-    u = dot3(tvec, pvec) * inv_det;
-    if (!(u >= 0.0f && u <= 1.0f)) return false;
-    f3 qvec = cross3(tvec, e1);
-    v = dot3(d, qvec) * inv_det;
-    if (!(v >= 0.0f && u + v <= 1.0f)) return false;
-    t = dot3(e2, qvec) * inv_det;
-    return t >= tmin;
-}
 
 }  // namespace vgi

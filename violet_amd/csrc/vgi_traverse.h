@@ -163,9 +163,9 @@ constexpr int32_t kTraversalDone = INT32_MIN;
 __device__ __forceinline__ bool is_leaf(int32_t link) { return (uint32_t)link > (uint32_t)kTraversalDone; }
 
 // One triangle against the ray, without branches (some lane of the wave
-// passes almost every test, so an early exit saves nothing): the arithmetic
-// and the conditions of Moller-Trumbore in vgi_bvh.h's intersect_tri; a zero
-// determinant makes u infinite or NaN and fails them.  Updates the hit if
+// passes almost every test, so an early exit saves nothing): Moller-Trumbore,
+// two-sided, in a fixed order of IEEE operations (the oracle's, bit for bit); a
+// zero determinant makes u infinite or NaN and fails the conditions.  Updates the hit if
 // this one is nearer (ties: the lower triangle id) and says whether it did.
 __device__ __forceinline__ bool closer_hit(f3 o, f3 d, Vf4 v0, Vf4 e1v, Vf4 e2v, float tmin, Hit& h) {
     const f3 e1 = mk3(e1v.x, e1v.y, e1v.z), e2 = mk3(e2v.x, e2v.y, e2v.z);

@@ -78,3 +78,19 @@ def test_scene_built_in_pieces(vgi, n_tris):
     d /= np.linalg.norm(d, axis=1, keepdims=True)
     rays = np.concatenate([o, np.full((m, 1), 5e-4), d, np.full((m, 1), 1000.0)], 1).astype(np.float32)
     assert _check(vgi, _soup(n_tris, 5), rays).any()
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("width,far", [(1.0, -900.0), (4.0, -4000.0)])
+def test_mixed_scales_lose_no_hit(vgi, width, far, axis):
+    """A small tiled surface at the edge of a node that spans a far triangle: the node's
+    rounding exceeds the surface's own padding, and the node's margin covers it."""
+    from test_traverse_replay import mixed_scale
+
+    from violet_amd import scene
+
+    pos, idx, rays = mixed_scale(width, far, axis, 60000, seed=2)
+    mesh = scene.Mesh(positions=pos, normals=np.tile(np.array([0, 0, 1], np.float32), (len(pos), 1)), indices=idx,
+                      tri_material=np.zeros(len(idx), np.uint32), albedo=np.full((1, 3), 0.5), metallic=np.zeros(1),
+                      roughness=np.full(1, 0.5))
+    assert _check(vgi, mesh, rays).mean() > 0.99

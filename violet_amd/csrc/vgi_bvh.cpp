@@ -78,9 +78,10 @@ inline int bins_for(int n) { return n >= 65536 ? 128 : n >= 2048 ? 64 : 32; }
 constexpr int kPiece = 16384;
 constexpr unsigned kBuildThreads = 8;
 // Largest vertex coordinate magnitude a scene may have: keeps every node's
-// grid step a float and the traversal's plane distances finite (the step
-// is below 2^34, so the stored step * 2^24 times |1/d| stays below 2^125
-// and q * step * |1/d| below 2^109 for |1/d| <= 1e20).
+// grid step a float and the traversal's plane distances finite (255 steps
+// span at most 2^41 and the margins, so the step is below 2^34, the stored
+// step * 2^24 times |1/d| stays below 2^125 and q * step * |1/d| below 2^109
+// for |1/d| <= 1e20).
 constexpr float kMaxCoord = 1099511627776.0f;  // 2^40
 constexpr int kMaxLeaf = 15;
 constexpr int kMedianDepth = 36;
@@ -370,6 +371,12 @@ struct Collapser {
         return idx;
     }
 
+    // The largest float at most x.
+    static float down(double x) {
+        const float f = (float)x;
+        return (double)f > x ? std::nextafter(f, -INFINITY) : f;
+    }
+
     // A float step s with x <= 255 * s, at least 2^-60.  Positions are
     // bounded by kMaxCoord, so x < 2^42 and s is a normal float.
     static double grid_step(double x) {
@@ -378,11 +385,18 @@ struct Collapser {
         return std::max((double)s, std::ldexp(1.0, -60));
     }
 
-    // The node's grid: per axis, the origin is the lowest used child plane
-    // and 255 steps reach the highest.  A child's lo rounds down and its hi
-    // up, so the quantised box contains the padded one (the divisions are in
-    // double, and the loops after them settle a quotient that rounding moved
-    // across a whole number).
+    // The node's grid: per axis, 255 steps span the children's padded boxes
+    // and a margin m on either side.  A child's lo rounds down and its hi up
+    // from its box widened by m, so its grid box keeps at least m between
+    // itself and the padded box (the divisions are in double, and the loops
+    // after them settle a quotient that rounding moved across a whole number).
+    // m covers what the traversal's plane distances err by on the scale of the
+    // node (slab_q: 2^-23 of its extent and 3 * 2^-24 of its origin), which
+    // the padding cannot: it goes with the child's own coordinates.  Without
+    // it, rays grazing a unit-sized floor whose node also held a triangle 900
+    // units away lost 104 of 100,000 hits.  On the scene of a million
+    // triangles rays visit as many nodes with it as without (camera rays
+    // 13.053, bounce rays 22.710 against 22.709, shadow rays 13.668).
     static void quantise(BvhNode& nd, const Box* box, const int32_t* child, int cnt) {
         bool used[4];
         for (int k = 0; k < 4; ++k) used[k] = k < cnt && child[k] != ~0;
@@ -394,14 +408,16 @@ struct Collapser {
                     hi = std::max(hi, box[k].hi[a]);
                 }
             if (!(lo <= hi)) lo = hi = 0.0f;  // no used child (cannot happen for a built tree)
-            const double s = grid_step((double)hi - (double)lo);
-            nd.org[a] = lo;
+            const double m = std::ldexp(std::max({(double)hi - (double)lo, std::fabs((double)lo), std::fabs((double)hi)}), -21);
+            const float org = down((double)lo - m);
+            const double s = grid_step((double)hi + m - (double)org);
+            nd.org[a] = org;
             nd.scale[a] = (float)std::ldexp(s, 24);  // see BvhNode::scale
             uint32_t qlo = 0, qhi = 0;
             for (int k = 0; k < 4; ++k) {
                 uint32_t l = 255u, h = 0u;  // unused: an empty interval
                 if (used[k]) {
-                    const double bl = (double)box[k].lo[a] - (double)lo, bh = (double)box[k].hi[a] - (double)lo;
+                    const double bl = (double)box[k].lo[a] - m - (double)org, bh = (double)box[k].hi[a] + m - (double)org;
                     l = (uint32_t)std::min(255.0, std::max(0.0, std::floor(bl / s)));
                     h = (uint32_t)std::min(255.0, std::max(0.0, std::ceil(bh / s)));
                     while (l > 0 && l * s > bl) --l;

@@ -12,15 +12,20 @@
  *           binary16 grid lines q * 2^-24 back into q), and four child
  *           links.  A child link >= 0
  *           is an inner node index; < 0 encodes a leaf ~((first << 4) | n).
- *           A child's quantised box contains its padded box (lo rounded
- *           down, hi rounded up).  An unused child has lo = 255, hi = 0 on
+ *           A child's quantised box contains its padded box and a margin
+ *           for the node's rounding (lo rounded down, hi rounded up).  An unused child has lo = 255, hi = 0 on
  *           every axis (an empty interval) and the empty leaf link ~0.
  *   tris  : leaf-ordered triangles as {v0, e1 = v1-v0, e2 = v2-v0} (3 x
  *           float4, 48 bytes); v0.w carries the scene triangle id.
- * Child boxes are padded by a small relative margin so the slab test is
- * conservative: a triangle the intersection routine accepts is never pruned
- * by its ancestors' boxes, and the closest hit (smallest t, ties to the
- * lowest triangle id) equals a brute-force loop over all triangles.
+ * Child boxes are padded, by 2^-16 of the child's coordinates (at least of 1)
+ * and 2^-21 of the node's (vgi_bvh.cpp), so that neither the rounding of the
+ * slab test (slab_q in vgi_traverse.h) nor that of the intersection routine
+ * prunes a triangle that the routine accepts: the closest hit (smallest t,
+ * ties to the lowest triangle id) equals a brute-force loop over all
+ * triangles.  Both roundings also grow with the distance to the ray's origin,
+ * which no stored box can cover: rays that start 300 units and more from
+ * geometry of a unit's size near the scene's origin can lose a grazing hit
+ * (about 70 of a million such rays, aimed at edges from 1000 units).
  *
  * Hit semantics follow violet: opaque, two-sided, t in [tmin, tmax];
  * shadow rays accept the first hit (RAY_FLAG_ACCEPT_FIRST_HIT_AND_END_SEARCH).
@@ -34,7 +39,7 @@
 namespace vgi {
 
 struct BvhNode {
-    float org[3];    // grid origin (at or below every used child's padded box)
+    float org[3];    // grid origin (below every used child's padded box)
     float scale[3];  // grid step per axis times 2^24 (255 steps span the node)
     uint32_t q[6];   // planes lo.x, hi.x, lo.y, hi.y, lo.z, hi.z: byte k = child k
     int32_t link[4];

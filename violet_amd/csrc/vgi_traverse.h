@@ -111,14 +111,16 @@ struct NodePlanes {
 // Slab interval [tn, tf] of child k of a quantised node, clipped to [tmin,
 // tmax]; the child is missed unless tn <= tf.  Per axis the distance to grid
 // line q is (q * 2^-24) * a + b with a = (step * 2^24) * idir and b =
-// (org - o) * idir; both scalings are by powers of two, so they add no
-// rounding to step * idir's, which moves a plane by at most 2^-24 of the
-// node's extent.  Against the exact
-// distance (org + q * step - o) * idir this errs by about an ulp of
-// |org - o| in world units plus the final rounding, inside the 2^-16
-// relative padding of every child box, so the test stays conservative.  An
-// unused child (lo = 255, hi = 0) has its near plane beyond its far one on
-// every axis.
+// (org - o) * idir.  In world units, with u = 2^-24, extent = 255 step and
+// plane = org + q * step, the distance errs by at most u * extent (rounding
+// of a) + 2 u |org - o| (of the difference and its product) + u |plane - o|
+// (of the sum), in all 2 u extent + 3 u (|org| + |o|), besides the relative
+// error of idir that all planes of the axis share.  The node's grid boxes
+// hold 8 u max(extent, |org|) beyond the padded ones (quantise); the rest, up
+// to 3 u |o|, is the padding's to cover (at least 256 u): it does for origins
+// within 85 units, and 85 times the child's own distance from the scene's
+// origin.  An unused child (lo = 255, hi = 0) has its near plane beyond its
+// far one on every axis.
 template <int k>
 __device__ __forceinline__ void slab_q(f3 a, f3 b, const NodePlanes& p, float tmin, float tmax, float& tn, float& tf) {
     const float tnx = __builtin_fmaf(qline<k>(p.nx01, p.nx23), a.x, b.x);

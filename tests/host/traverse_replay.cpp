@@ -1,12 +1,16 @@
 // Replays the device traversal (vgi_traverse.h) on the CPU over the nodes that
-// the scene builder makes, the node's slab test in the device's float
-// operations, against a brute-force loop over all triangles.
+// the scene builder makes: a wave of 64 rays in lockstep with its traversal
+// stack in a 20-entry "LDS" part and a private part, the node's slab test in
+// the device's float operations, against a brute-force loop over all
+// triangles.  Reports the rays whose closest hit differs from the loop's and
+// how the stacks grew; an access outside a stack ends the program.
 //
 //   traverse_replay <file>   file: u32 vertices, triangles, rays; f32 positions
 //                            [v][3]; u32 indices [t][3]; f32 rays [r][8]
-// Prints: rays, hits, lost (closest hit differs from the loop's, bit for bit),
-// any (any-hit answer differs).
-#include <algorithm>
+// Prints: rays, hits, lost (closest hit differs), any (any-hit answer differs),
+// the most stack entries of a lane, the most moves to private memory of a lane,
+// node steps of all waves, how many of them did stack moves, and how many of
+// those had a lane with entries to move.
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -20,6 +24,9 @@
 using namespace vgi;
 
 namespace {
+
+constexpr int32_t kDone = INT32_MIN;
+bool is_leaf(int32_t l) { return (uint32_t)l > (uint32_t)kDone; }
 
 void require(bool ok, const char* what) {
     if (!ok) {
@@ -50,51 +57,158 @@ bool closer_hit(f3 o, f3 d, const BvhTri& tr, float tmin, RayHit& h) {
     return true;
 }
 
-struct Ray {
+struct Totals {
+    long long steps = 0, move_steps = 0, needed_steps = 0;
+    int max_entries = 0, max_moves = 0;
+} totals;
+
+struct Lane {
+    bool used = false;
     f3 o, d;
     float id[3], tmin;
     bool pos[3];
+    RayHit h;
+    int32_t node, leaf = 0;
+    uint32_t base, p;
+    int32_t lds[kLdsStackEntries];
+    int32_t spill[kStackMaxEntries];
+    int spilled = 0, moves = 0;
+    int32_t& at(uint32_t a) {
+        const uint32_t off = a - base;
+        require(off % kStackStride == 0 && off / kStackStride < kLdsStackEntries, "LDS stack access out of range");
+        return lds[off / kStackStride];
+    }
+    void entries() {
+        const int n = (int32_t)(p - base) / (int32_t)kStackStride + spilled;
+        if (n > totals.max_entries) totals.max_entries = n;
+    }
 };
 
 float safe_dir(float v) { return std::fabs(v) < 1e-20f ? std::copysign(1e-20f, v) : v; }
 
 // The slab test of child k (slab_q): true if hit, with its entry distance.
-bool slab(const Ray& r, const BvhNode& n, int k, float tmax, float& tn) {
-    const float o[3] = {r.o.x, r.o.y, r.o.z};
-    float tns[3], tfs[3];
+bool slab(const Lane& l, const BvhNode& n, int k, float& tn) {
+    const float o[3] = {l.o.x, l.o.y, l.o.z};
+    float near = l.tmin, far = l.h.t, tns[3], tfs[3];
     for (int a = 0; a < 3; ++a) {
-        const float sa = n.scale[a] * r.id[a];
-        const float sb = (n.org[a] - o[a]) * r.id[a];
+        const float sa = n.scale[a] * l.id[a];
+        const float sb = (n.org[a] - o[a]) * l.id[a];
         const uint32_t lo = (n.q[2 * a] >> (8 * k)) & 255u, hi = (n.q[2 * a + 1] >> (8 * k)) & 255u;
         const float ql = std::ldexp((float)lo, -24), qh = std::ldexp((float)hi, -24);
-        tns[a] = std::fmaf(r.pos[a] ? ql : qh, sa, sb);
-        tfs[a] = std::fmaf(r.pos[a] ? qh : ql, sa, sb);
+        tns[a] = std::fmaf(l.pos[a] ? ql : qh, sa, sb);
+        tfs[a] = std::fmaf(l.pos[a] ? qh : ql, sa, sb);
     }
-    tn = std::fmax(std::fmax(std::fmax(tns[0], tns[1]), tns[2]), r.tmin);
-    return tn <= std::fmin(std::fmin(std::fmin(tfs[0], tfs[1]), tfs[2]), tmax);
+    near = std::fmax(std::fmax(std::fmax(tns[0], tns[1]), tns[2]), near);
+    far = std::fmin(std::fmin(std::fmin(tfs[0], tfs[1]), tfs[2]), far);
+    tn = near;
+    return near <= far;
 }
 
-// Nearest child first, or, for any hit, in any order.
-RayHit traverse(const HostScene& s, const Ray& r, RayHit h, bool any) {
-    std::vector<int32_t> stack{s.root};
-    while (!stack.empty()) {
-        const int32_t l = stack.back();
-        stack.pop_back();
-        if (l < 0) {
-            const uint32_t enc = ~(uint32_t)l, first = enc >> 4, n = enc & 15u;
-            for (uint32_t k = 0; k < n; ++k)
-                if (closer_hit(r.o, r.d, s.tris[first + k], r.tmin, h) && any) return h;
-            continue;
-        }
-        const BvhNode& n = s.nodes[l];
-        float tn[4];
-        int order[4], cnt = 0;
-        for (int k = 0; k < 4; ++k)
-            if (slab(r, n, k, h.t, tn[k])) order[cnt++] = k;
-        std::sort(order, order + cnt, [&](int i, int j) { return tn[i] > tn[j]; });
-        for (int i = 0; i < cnt; ++i) stack.push_back(n.link[order[i]]);
+template <bool kAny>
+void run_wave(const HostScene& s, std::vector<Lane>& w) {
+    for (Lane& l : w) {
+        l.p = l.base;
+        l.at(l.p) = kDone;
+        l.at(l.p + kStackStride) = kDone;
+        l.node = s.root;
     }
-    return h;
+    for (;;) {
+        int n_leaf = 0, n_want = 0;
+        for (const Lane& l : w) {
+            if (!l.used) continue;
+            n_leaf += l.leaf != 0;
+            n_want += l.node >= 0 && l.leaf == 0;
+        }
+        if (n_want != 0 && 3 * n_want >= 2 * n_leaf) {
+            ++totals.steps;
+            uint64_t inner = 0, over = 0;
+            bool need = false;
+            for (size_t k = 0; k < w.size(); ++k) {
+                const Lane& l = w[k];
+                if (!l.used) continue;
+                inner |= (uint64_t)(l.node >= 0) << k;
+                over |= (uint64_t)stack_over(l.p, l.base) << k;
+                need |= l.node >= 0 && (int32_t)(l.p - l.base) > (int32_t)(kStackStride * (kLdsStackEntries - 6));
+            }
+            totals.move_steps += full_stacks(inner, over) != 0;
+            totals.needed_steps += need;
+            for (Lane& l : w) {
+                if (!l.used || l.node < 0) continue;
+                if (stack_over(l.p, l.base)) {
+                    require(l.spilled + kSpillEntries <= (int)kStackMaxEntries, "private stack full");
+                    for (int k = 0; k < kSpillEntries; ++k) l.spill[l.spilled + k] = l.at(l.base + kStackStride * (2 + k));
+                    l.spilled += kSpillEntries;
+                    l.p -= kStackStride * kSpillEntries;
+                    for (uint32_t q = l.base + kStackStride * 2; q <= l.p + kStackStride; q += kStackStride)
+                        l.at(q) = l.at(q + kStackStride * kSpillEntries);
+                    if (++l.moves > totals.max_moves) totals.max_moves = l.moves;
+                }
+                const BvhNode& n = s.nodes[l.node];
+                float tn[4];
+                bool hit[4];
+                int order[4] = {0, 1, 2, 3}, cnt = 0;
+                for (int k = 0; k < 4; ++k) {
+                    hit[k] = slab(l, n, k, tn[k]);
+                    cnt += hit[k];
+                }
+                if (!kAny)  // farther first, missed children last
+                    for (int i = 0; i < 3; ++i)
+                        for (int j = i + 1; j < 4; ++j) {
+                            const float ti = hit[order[i]] ? tn[order[i]] : -INFINITY;
+                            const float tj = hit[order[j]] ? tn[order[j]] : -INFINITY;
+                            if (tj > ti) std::swap(order[i], order[j]);
+                        }
+                if (kAny) {
+                    for (int k = 0; k < 4; ++k) {
+                        l.at(l.p + 2 * kStackStride) = n.link[k];
+                        l.p += hit[k] ? kStackStride : 0u;
+                    }
+                } else {
+                    for (int k = 0; k < 4; ++k) l.at(l.p + (2 + k) * kStackStride) = n.link[order[k]];
+                    l.p += kStackStride * cnt;
+                }
+                l.entries();
+                const int32_t e0 = l.at(l.p + kStackStride), e1 = l.at(l.p);
+                const bool aside = l.leaf == 0 && is_leaf(e0);
+                l.leaf = aside ? e0 : l.leaf;
+                l.node = aside ? e1 : e0;
+                l.p -= aside ? 2 * kStackStride : kStackStride;
+            }
+        } else if (n_leaf != 0) {
+            for (Lane& l : w) {
+                if (!l.used || l.leaf == 0) continue;
+                const uint32_t enc = ~(uint32_t)l.leaf, first = enc >> 4, n = enc & 15u;
+                bool got = false;
+                for (uint32_t k = 0; k < n && !(kAny && got); ++k)
+                    got = closer_hit(l.o, l.d, s.tris[first + k], l.tmin, l.h) || (!kAny && got);
+                l.leaf = 0;
+                if (kAny && got) {
+                    l.node = kDone;
+                    l.spilled = 0;
+                } else if (is_leaf(l.node)) {
+                    l.leaf = l.node;
+                    l.node = l.at(l.p + kStackStride);
+                    l.p -= kStackStride;
+                }
+            }
+        } else {
+            bool back = false;
+            for (Lane& l : w)
+                if (l.used && l.spilled > 0) {
+                    l.spilled -= kSpillEntries;
+                    for (int k = 0; k < kSpillEntries; ++k) l.at(l.base + kStackStride * (2 + k)) = l.spill[l.spilled + k];
+                    l.p = l.base + kStackStride * (kSpillEntries - 1);
+                    l.node = l.at(l.p + 2 * kStackStride);
+                    if (is_leaf(l.node)) {
+                        l.leaf = l.node;
+                        l.node = l.at(l.p + kStackStride);
+                        l.p -= kStackStride;
+                    }
+                    back = true;
+                }
+            if (!back) break;
+        }
+    }
 }
 
 template <class T>
@@ -127,21 +241,43 @@ int main(int argc, char** argv) {
     require(build_scene_host(&desc, s) == VGI_OK, "scene refused");
 
     long long hits = 0, lost = 0, any = 0;
-    for (uint32_t k = 0; k < n[2]; ++k) {
-        const float* q = rays.data() + 8 * (size_t)k;
-        Ray r{mk3(q[0], q[1], q[2]), mk3(q[4], q[5], q[6]), {}, q[3], {}};
-        for (int a = 0; a < 3; ++a) {
-            r.id[a] = 1.0f / safe_dir(q[4 + a]);
-            r.pos[a] = r.id[a] >= 0.0f;
+    for (uint32_t r0 = 0; r0 < n[2]; r0 += 64) {
+        std::vector<Lane> w(64);
+        for (uint32_t k = 0; k < 64; ++k) {
+            Lane& l = w[k];
+            l.base = 4 * k;  // LDS byte address of the lane's slot 0 in a kernel without other LDS
+            l.used = r0 + k < n[2];
+            if (!l.used) continue;
+            const float* r = rays.data() + 8 * (size_t)(r0 + k);
+            l.o = mk3(r[0], r[1], r[2]);
+            l.d = mk3(r[4], r[5], r[6]);
+            l.tmin = r[3];
+            l.h = RayHit{r[7], 0.0f, 0.0f, 0xFFFFFFFFu};
+            for (int a = 0; a < 3; ++a) {
+                l.id[a] = 1.0f / safe_dir(r[4 + a]);
+                l.pos[a] = l.id[a] >= 0.0f;
+            }
         }
-        const RayHit miss{q[7], 0.0f, 0.0f, 0xFFFFFFFFu};
-        RayHit brute = miss;
-        for (const BvhTri& t : s.tris) closer_hit(r.o, r.d, t, r.tmin, brute);
-        const RayHit h = traverse(s, r, miss, false);
-        hits += brute.tri != miss.tri;
-        lost += std::memcmp(&h, &brute, sizeof(RayHit)) != 0;
-        any += (brute.tri != miss.tri) != (traverse(s, r, miss, true).tri != miss.tri);
+        std::vector<RayHit> brute(64);
+        for (int k = 0; k < 64; ++k) {
+            brute[k] = w[k].h;
+            if (w[k].used)
+                for (const BvhTri& t : s.tris) closer_hit(w[k].o, w[k].d, t, w[k].tmin, brute[k]);
+        }
+        std::vector<Lane> wa = w;
+        run_wave<false>(s, w);
+        run_wave<true>(s, wa);
+        for (int k = 0; k < 64; ++k) {
+            if (!w[k].used) continue;
+            const bool hit = brute[k].tri != 0xFFFFFFFFu;
+            hits += hit;
+            lost += std::memcmp(&w[k].h, &brute[k], sizeof(RayHit)) != 0;
+            any += hit != (wa[k].h.tri != 0xFFFFFFFFu);
+        }
     }
-    std::printf("rays %u hits %lld lost %lld any %lld\n", n[2], hits, lost, any);
+    std::printf("rays %u hits %lld lost %lld any %lld max_entries %d max_moves %d steps %lld move_steps %lld "
+                "needed_steps %lld nodes %zu\n",
+                n[2], hits, lost, any, totals.max_entries, totals.max_moves, totals.steps, totals.move_steps,
+                totals.needed_steps, s.nodes.size());
     return 0;
 }

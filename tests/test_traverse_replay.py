@@ -1,9 +1,11 @@
-"""The BVH's boxes against the traversal's rounding, on the CPU: the nodes of
-the scene builder, with the device's slab test replayed in its float
-operations, give the closest hit of a brute-force loop bit for bit, on scenes
-that mix scales (a small tiled surface near the origin and one triangle far
-away), where a node's rounding errors are larger than the padding of a child
-near the origin."""
+"""The traversal on the CPU, over the nodes of the scene builder: waves of 64
+rays in lockstep with the device's stack and the slab test's float operations.
+
+* The closest hit is a brute-force loop's bit for bit on scenes that mix
+  scales (a small tiled surface near the origin and one triangle far away),
+  where a node's rounding errors are larger than the padding of a child near
+  the origin.
+* Stacks move to private memory when they are full and at no other step."""
 from __future__ import annotations
 
 import shutil
@@ -77,3 +79,23 @@ def test_mixed_scales_lose_no_hit(replay, width, far, axis):
     r = replay(*mixed_scale(width, far, axis, 60000, seed=2))
     assert r["hits"] > 0.99 * r["rays"]
     assert r["lost"] == 0 and r["any"] == 0, r
+
+
+def soup(n, seed):
+    rng = np.random.default_rng(seed)
+    pos = (rng.uniform(-1.0, 1.0, (n, 1, 3)) + rng.normal(0, 0.4 / n ** (1 / 3), (n, 3, 3))).reshape(-1, 3)
+    return pos.astype(np.float32), np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+
+
+def test_only_full_stacks_move(replay):
+    """A wave's node steps look into its stacks only when a lane's is full, not whenever one of
+    its lanes is done."""
+    rng = np.random.default_rng(3)
+    m = 6400
+    o = rng.uniform(-2.0, 2.0, (m, 3))
+    d = rng.uniform(-1.0, 1.0, (m, 3)) - o
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.concatenate([o, np.full((m, 1), 5e-4), d, np.full((m, 1), 1000.0)], 1)
+    r = replay(*soup(2000, 7), rays)
+    assert r["lost"] == 0 and r["any"] == 0 and r["max_moves"] == 0
+    assert r["steps"] > 0 and r["move_steps"] == r["needed_steps"] == 0, r

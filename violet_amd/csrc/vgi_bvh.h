@@ -112,6 +112,17 @@ constexpr int kBvhMaxDepth = 64;     // binary build depth bound (the 4-wide tre
 constexpr uint32_t kLdsStackEntries = 20;
 constexpr int kSpillEntries = 8;
 constexpr uint32_t kStackMaxEntries = 3 * kBvhMaxDepth;  // 3 far children per 4-wide level
+constexpr uint32_t kStackStride = 64 * sizeof(int32_t);  // LDS bytes from one entry of a lane to the next
+// A node step writes up to p + 5 kStackStride, where p is the byte address
+// below the lane's top entry: past the LDS part beyond its slot
+// kLdsStackEntries - 6.
+VGI_HD bool stack_over(uint32_t p, uint32_t base) { return p > base + kStackStride * (kLdsStackEntries - 6u); }
+// The lanes of a wave that move entries to private memory before a node step:
+// those at a node (`inner`) whose stack is `over`.  A lane that popped its last
+// sentinel is over too: it holds p = base - kStackStride, which wraps for a
+// base near zero.  Without the mask every step after a wave's first lane was
+// done took the branch of a full stack.
+VGI_HD uint64_t full_stacks(uint64_t inner, uint64_t over) { return inner & over; }
 
 // Register budget of the per-pixel ray-tracing kernels, as waves per SIMD:
 // 6, 7 and 8 are within 3% of each other (64 registers spill a few values

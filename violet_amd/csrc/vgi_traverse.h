@@ -232,9 +232,9 @@ __device__ __forceinline__ Hit traverse(const SceneView& s, f3 o, f3 d, float tm
     uint32_t p = base;
     lds_at(p) = kTraversalDone;
     lds_at(p + 256u) = kTraversalDone;
-    // A step writes up to p + 1280.  Beyond `limit` that would leave the LDS
-    // part: the lane's oldest entries then move to private memory.
-    const uint32_t limit = base + 256u * (kLdsStackEntries - 6u);
+    // A step writes up to p + 1280.  Where that would leave the LDS part
+    // (stack_over) the lane's oldest entries move to private memory.
+    static_assert(kStackStride == 256u, "the offsets below");
     int32_t spill[kStackMaxEntries];
     int32_t spilled = 0;
     // Every step of the wave moves at least one lane, and each node and leaf
@@ -245,11 +245,11 @@ __device__ __forceinline__ Hit traverse(const SceneView& s, f3 o, f3 d, float tm
     bool live = true;
     while (live) {
         const bool inner = node >= 0;
-        const uint64_t m_leaf = __ballot(leaf != 0);
-        const uint64_t m_want = __ballot(inner) & ~m_leaf;
+        const uint64_t m_inner = __ballot(inner), m_leaf = __ballot(leaf != 0);
+        const uint64_t m_want = m_inner & ~m_leaf;
         if (m_want != 0 && 3 * (int)__popcll(m_want) >= 2 * (int)__popcll(m_leaf)) {
-            if (__ballot(p > limit) != 0) {  // rare: a stack of more than kLdsStackEntries - 6 entries
-                if (inner && p > limit) {
+            if (full_stacks(m_inner, __ballot(stack_over(p, base))) != 0) {  // rare
+                if (inner && stack_over(p, base)) {
                     if (spilled + kSpillEntries <= (int32_t)kStackMaxEntries) {
                         for (int k = 0; k < kSpillEntries; ++k) spill[spilled + k] = lds_at(base + 256u * (2 + k));
                         spilled += kSpillEntries;

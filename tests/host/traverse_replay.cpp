@@ -9,8 +9,9 @@
 //                            [v][3]; u32 indices [t][3]; f32 rays [r][8]
 // Prints: rays, hits, lost (closest hit differs), any (any-hit answer differs),
 // the most stack entries of a lane, the most moves to private memory of a lane,
-// node steps of all waves, how many of them did stack moves, and how many of
-// those had a lane with entries to move.
+// node steps of all waves, how many of them did stack moves, how many had a
+// lane with entries to move, and the lanes that sat out a node step because all
+// they had left was in private memory.
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -60,6 +61,7 @@ bool closer_hit(f3 o, f3 d, const BvhTri& tr, float tmin, RayHit& h) {
 struct Totals {
     long long steps = 0, move_steps = 0, needed_steps = 0;
     int max_entries = 0, max_moves = 0;
+    long long idle = 0;
 } totals;
 
 struct Lane {
@@ -104,6 +106,9 @@ bool slab(const Lane& l, const BvhNode& n, int k, float& tn) {
     return near <= far;
 }
 
+// Nothing left but entries in private memory.
+bool waits(const Lane& l) { return l.used && l.spilled > 0 && l.node == kDone && l.leaf == 0; }
+
 template <bool kAny>
 void run_wave(const HostScene& s, std::vector<Lane>& w) {
     for (Lane& l : w) {
@@ -112,7 +117,21 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
         l.at(l.p + kStackStride) = kDone;
         l.node = s.root;
     }
+    bool deep = false;
     for (;;) {
+        if (deep)
+            for (Lane& l : w)
+                if (waits(l)) {
+                    l.spilled -= kSpillEntries;
+                    for (int k = 0; k < kSpillEntries; ++k) l.at(l.base + kStackStride * (2 + k)) = l.spill[l.spilled + k];
+                    l.p = l.base + kStackStride * (kSpillEntries - 1);
+                    l.node = l.at(l.p + 2 * kStackStride);
+                    if (is_leaf(l.node)) {
+                        l.leaf = l.node;
+                        l.node = l.at(l.p + kStackStride);
+                        l.p -= kStackStride;
+                    }
+                }
         int n_leaf = 0, n_want = 0;
         for (const Lane& l : w) {
             if (!l.used) continue;
@@ -126,6 +145,7 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
             for (size_t k = 0; k < w.size(); ++k) {
                 const Lane& l = w[k];
                 if (!l.used) continue;
+                totals.idle += waits(l);
                 inner |= (uint64_t)(l.node >= 0) << k;
                 over |= (uint64_t)stack_over(l.p, l.base) << k;
                 need |= l.node >= 0 && (int32_t)(l.p - l.base) > (int32_t)(kStackStride * (kLdsStackEntries - 6));
@@ -138,9 +158,11 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
                     require(l.spilled + kSpillEntries <= (int)kStackMaxEntries, "private stack full");
                     for (int k = 0; k < kSpillEntries; ++k) l.spill[l.spilled + k] = l.at(l.base + kStackStride * (2 + k));
                     l.spilled += kSpillEntries;
+                    deep = true;
                     l.p -= kStackStride * kSpillEntries;
-                    for (uint32_t q = l.base + kStackStride * 2; q <= l.p + kStackStride; q += kStackStride)
-                        l.at(q) = l.at(q + kStackStride * kSpillEntries);
+                    constexpr int kRest = kLdsStackEntries - 2 - kSpillEntries;
+                    for (int k = 0; k < kRest; ++k)
+                        l.at(l.base + kStackStride * (2 + k)) = l.at(l.base + kStackStride * (2 + kSpillEntries + k));
                     if (++l.moves > totals.max_moves) totals.max_moves = l.moves;
                 }
                 const BvhNode& n = s.nodes[l.node];
@@ -192,23 +214,10 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
                 }
             }
         } else {
-            bool back = false;
-            for (Lane& l : w)
-                if (l.used && l.spilled > 0) {
-                    l.spilled -= kSpillEntries;
-                    for (int k = 0; k < kSpillEntries; ++k) l.at(l.base + kStackStride * (2 + k)) = l.spill[l.spilled + k];
-                    l.p = l.base + kStackStride * (kSpillEntries - 1);
-                    l.node = l.at(l.p + 2 * kStackStride);
-                    if (is_leaf(l.node)) {
-                        l.leaf = l.node;
-                        l.node = l.at(l.p + kStackStride);
-                        l.p -= kStackStride;
-                    }
-                    back = true;
-                }
-            if (!back) break;
+            break;
         }
     }
+    for (const Lane& l : w) require(!l.used || l.spilled == 0, "a lane ended with entries in private memory");
 }
 
 template <class T>
@@ -276,8 +285,8 @@ int main(int argc, char** argv) {
         }
     }
     std::printf("rays %u hits %lld lost %lld any %lld max_entries %d max_moves %d steps %lld move_steps %lld "
-                "needed_steps %lld nodes %zu\n",
+                "needed_steps %lld idle %lld nodes %zu\n",
                 n[2], hits, lost, any, totals.max_entries, totals.max_moves, totals.steps, totals.move_steps,
-                totals.needed_steps, s.nodes.size());
+                totals.needed_steps, totals.idle, s.nodes.size());
     return 0;
 }

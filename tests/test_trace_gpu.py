@@ -98,9 +98,10 @@ def _onion(n_quads, seed):
 
 def test_deep_traversal_stack_spills_exactly(vgi):
     """Rays through 25000 stacked quads hit every box on their way down, so
-    their traversal stacks grow past the 16 entries kept in LDS (to 21 on this
-    scene, by a host simulation of the traversal) into private memory; hits
-    must still equal the brute-force loop bit for bit, also for oblique rays."""
+    their traversal stacks grow past the 14 entries kept in LDS (to 26 on this
+    scene; test_traverse_replay.py checks that they do) into private memory;
+    hits must still equal the brute-force loop bit for bit, also for oblique
+    rays."""
     import oracle
     from violet_amd import scene
 

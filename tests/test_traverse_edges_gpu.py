@@ -55,7 +55,8 @@ def test_edges(vgi, n_tris, copies, n_rays, interval):
 
 def test_stack_leaves_lds_twice(vgi):
     """200,000 stacked quads: every box on a ray's way is hit, three children
-    stay on the stack per level, about 30 entries: two moves of eight."""
+    stay on the stack per level, about 30 entries: two moves of eight
+    (test_traverse_replay.py checks that there are as many)."""
     rng = np.random.default_rng(8)
     m = 256
     o = np.column_stack([rng.uniform(-0.5, 0.5, (m, 2)), np.where(rng.random(m) < 0.5, -1.0, 11.0)])

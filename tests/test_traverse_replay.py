@@ -5,7 +5,10 @@ rays in lockstep with the device's stack and the slab test's float operations.
   scales (a small tiled surface near the origin and one triangle far away),
   where a node's rounding errors are larger than the padding of a child near
   the origin.
-* Stacks move to private memory when they are full and at no other step."""
+* Stacks move to private memory when they are full and at no other step, and a
+  lane whose LDS part is empty goes on with what it moved without waiting for
+  the rest of its wave.  The scenes of the GPU tests that mean to do so do
+  leave LDS."""
 from __future__ import annotations
 
 import shutil
@@ -99,3 +102,30 @@ def test_only_full_stacks_move(replay):
     r = replay(*soup(2000, 7), rays)
     assert r["lost"] == 0 and r["any"] == 0 and r["max_moves"] == 0
     assert r["steps"] > 0 and r["move_steps"] == r["needed_steps"] == 0, r
+
+
+def piled_rays(m, seed, kind):
+    """Rays at a pile of quads over z in [0, 10]: along it from both ends, or from inside in all directions."""
+    rng = np.random.default_rng(seed)
+    up = rng.random(m) < 0.5
+    o = np.column_stack([rng.uniform(-0.5, 0.5, (m, 2)), np.where(up, -1.0, 11.0)])
+    d = np.column_stack([rng.normal(0, 0.02, (m, 2)), np.where(up, 1.0, -1.0)])
+    if kind == "inside":
+        o[:, 2] = rng.uniform(0.0, 10.0, m)
+        d = rng.standard_normal((m, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    return np.concatenate([o, np.full((m, 1), 5e-4), d, np.full((m, 1), 1000.0)], 1)
+
+
+@pytest.mark.parametrize("kind", ["along", "inside"])
+@pytest.mark.parametrize("quads,moves", [(25_000, 1), (200_000, 2)])
+def test_deep_stacks_go_on_alone(replay, quads, moves, kind):
+    """The piles of test_deep_traversal_stack_spills_exactly and test_stack_leaves_lds_twice."""
+    from test_trace_gpu import _onion
+
+    mesh = _onion(quads, 4)
+    r = replay(mesh.positions, mesh.indices, piled_rays(256, 8, kind))
+    assert r["lost"] == 0 and r["any"] == 0
+    assert r["max_entries"] > 14 and r["max_moves"] >= moves, r
+    assert r["move_steps"] == r["needed_steps"] > 0
+    assert r["idle"] == 0, r

@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes as C
 import re
+import struct
 import subprocess
 from pathlib import Path
 
@@ -66,3 +67,26 @@ def test_invalid_arguments_return_status_and_message():
     out = C.c_void_p()
     assert lib.vgi_denoiser_create(0, 0, 0, None, C.byref(out)) == _lib.VGI_E_INVALID
     assert out.value is None
+
+
+@pytest.mark.parametrize("name,has_pc", [("ind_diff_sample_gen", True), ("ind_diff_sample_validate", False),
+                                         ("ind_spec_sample_gen", True), ("ind_spec_sample_validate", False)])
+def test_sample_passes_name_themselves_in_their_errors(name, has_pc):
+    from violet_amd import _lib
+
+    lib = _lib.lib()
+    fn = getattr(lib, f"vgi_pass_{name}")
+    fp, rt = C.create_string_buffer(4096), C.create_string_buffer(4096)  # zeros: F32 storage, no scene
+
+    def call(w, h, storage):
+        io = C.create_string_buffer(struct.pack("<3I", w, h, storage), 4096)
+        pc = [C.cast(C.create_string_buffer(64), fn.argtypes[3])] if has_pc else []
+        args = [C.cast(b, t) for b, t in zip((fp, rt, io), fn.argtypes)]
+        assert fn(*args, *pc, None) == _lib.VGI_E_INVALID
+        return lib.vgi_last_error().decode()
+
+    assert call(0, 16, 0) == f"vgi_pass_{name}: bad size"
+    assert call(16, 16, 1) == f"vgi_pass_{name}: storage mismatch"
+    assert call(16, 16, 0) == f"vgi_pass_{name}: missing binding"
+    assert fn(*[None] * len(fn.argtypes)) == _lib.VGI_E_INVALID
+    assert lib.vgi_last_error().decode() == f"vgi_pass_{name}: null argument"

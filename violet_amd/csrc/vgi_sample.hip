@@ -457,6 +457,15 @@ struct BatchMinWaves<JobSpecRays<S>> {
     static constexpr int value = kTraceWaves;
 };
 
+static const char* sample_pass_name(uint32_t pass) {
+    switch (pass) {
+        case kSampleSpecValidate: return "ind_spec_sample_validate";
+        case kSampleDiffGen: return "ind_diff_sample_gen";
+        case kSampleDiffValidate: return "ind_diff_sample_validate";
+        default: return "ind_spec_sample_gen";
+    }
+}
+
 // What the entry points of the single passes check, for each pass of a set;
 // its trace resources and its image size.
 static vgi_status check_sample_set(const vgi_trace_resources* tr, const SampleSet& a, TraceRes& t, uint32_t& w,
@@ -497,9 +506,10 @@ static vgi_status check_sample_set(const vgi_trace_resources* tr, const SampleSe
                 break;
             }
         }
-        VGI_REQUIRE(valid_dims(pw, ph), "sample rays: bad size");
-        VGI_REQUIRE(tr && storage == tr->storage, "sample rays: storage mismatch");
-        VGI_REQUIRE(bound, "sample rays: missing binding");
+        const char* name = sample_pass_name(a.pass[k]);
+        VGI_REQUIRE(valid_dims(pw, ph), "vgi_pass_%s: bad size", name);
+        VGI_REQUIRE(storage == tr->storage, "vgi_pass_%s: storage mismatch", name);
+        VGI_REQUIRE(bound, "vgi_pass_%s: missing binding", name);
         VGI_REQUIRE(k == 0 || (pw == w && ph == h), "internal: sample passes of different sizes");
         w = pw;
         h = ph;

@@ -79,7 +79,15 @@ vgi_status vgi_fence_wait(vgi_fence* fence, uint32_t timeout_ms, double* waited_
  * pass by render_graph.rs:2585-2591,2664-2669).  When enabled, every pass
  * entry point records a hipEvent pair around its kernel(s) on its stream.
  * vgi_profiler_read() waits for the recorded events, accumulates them per
- * pass name and returns up to `cap` entries. */
+ * pass name and returns up to `cap` entries.
+ *
+ * A frame runs each lobe's sample passes (vgi_pass_ind_{diff,spec}_sample_gen
+ * and _validate) as one launch, but as one each while the timers take one of
+ * them (every pass, or vgi_profiler_only with its name) or the traversal
+ * statistics are on, so that each has its own entry; a batch likewise
+ * ("batch_ind_diff_sample_gen", ...; not a captured one, whose launches are
+ * not timed).  Results are the same; the frame takes longer.  The shared
+ * launches are "ind_diff_sample" and "ind_spec_sample" ("batch_..."). */
 typedef struct vgi_profile_entry {
     char name[48];
     double total_ms;     /* summed kernel time */

@@ -55,13 +55,17 @@ static const char* kind_name(int kind) {
 struct vgi_batch {
     vgi_batch_config cfg{};
     size_t offsets[kSlotCount] = {};
-    size_t arena_bytes = 0;
+    size_t arena_bytes = 0, unsplit_bytes = 0;  // of all tables; without those of split lobes
     void* host[2] = {nullptr, nullptr};
     void* dev[2] = {nullptr, nullptr};
     hipEvent_t done[2] = {nullptr, nullptr};
     bool used[2] = {false, false};
     int flip = 0;
     std::vector<RecordSink> recs;
+    // Under the per-pass timers a lobe's generation and validation run as a
+    // launch each: their records, one part each, for the lobe's two slots.
+    bool split = false;
+    std::vector<PassRec> parts;
     hipStream_t cap = nullptr;  // capture/replay stream (graph mode)
     hipEvent_t ev_in = nullptr;
     // second lane (concurrent_lanes): independent slot chains beside the main stream
@@ -124,7 +128,14 @@ extern "C" vgi_status vgi_batch_create(const vgi_batch_config* cfg, vgi_batch** 
     if (!b) return set_error(VGI_E_NOMEM, "vgi_batch_create: out of host memory");
     b->cfg = c;
     size_t off = 0;
-    for (int s = 0; s < kSlotCount; ++s) {
+    // the slots of split lobes last: their tables are uploaded only when used
+    int order[kSlotCount], k = 0;
+    for (int s = 0; s < kSlotCount; ++s)
+        if (s != kSlotTimedSpec && s != kSlotTimedDiff) order[k++] = s;
+    order[k++] = kSlotTimedSpec;
+    order[k++] = kSlotTimedDiff;
+    for (int s : order) {
+        if (s == kSlotTimedSpec) b->unsplit_bytes = off;
         const BatchOps* o = batch_ops(slot_kind(s));
         if (!o) {
             delete b;
@@ -154,6 +165,7 @@ extern "C" vgi_status vgi_batch_create(const vgi_batch_config* cfg, vgi_batch** 
         return check_hip(e, "vgi_batch_create");
     }
     b->recs.resize(c.max_views);
+    b->parts.resize(c.max_views);
     *out = b;
     return VGI_OK;
 }
@@ -173,22 +185,56 @@ static uint32_t groups_for(const vgi_batch* b, int slot, const BatchOps* o) {
     return g ? g : b->grid_bound[slot];
 }
 
+// The part of a lobe that a slot launches when the timers take its passes
+// apart; kSamplePassCount for every other slot.
+static uint32_t split_part(int slot) {
+    switch (slot) {
+        case kSlotSampleSpec: return kSampleSpecValidate;
+        case kSlotTimedSpec: return kSampleSpecGen;
+        case kSlotSampleDiff: return kSampleDiffGen;
+        case kSlotTimedDiff: return kSampleDiffValidate;
+        default: return kSamplePassCount;
+    }
+}
+
+// A slot's records, one per view that issues it, to `list`; their number.
+static int slot_records(vgi_batch* b, int slot, uint32_t num_views, const PassRec** list) {
+    const uint32_t part = b->split ? split_part(slot) : (uint32_t)kSamplePassCount;
+    const int from = part == kSampleSpecGen ? kSlotSampleSpec : part == kSampleDiffValidate ? kSlotSampleDiff : slot;
+    int n = 0;
+    for (uint32_t v = 0; v < num_views; ++v) {
+        if (!b->recs[v].has[from]) continue;
+        const PassRec* r = &b->recs[v].recs[from];
+        if (part != kSamplePassCount) {
+            PassRec& one = b->parts[v];
+            one = *r;
+            if (!one.io.sample.keep((SamplePass)part)) continue;
+            r = &one;
+        }
+        list[n++] = r;
+    }
+    return n;
+}
+
 // Upload of the arena and every slot's launch on `main` and the side lane
 // (all slots in graph mode, so the captured topology never changes; only
 // occupied ones otherwise), joined back into `main` at the end.
 static vgi_status issue_slots(vgi_batch* b, int a, uint32_t storage, size_t lds, Lanes& lanes, bool all_slots,
                               bool profile) {
-    VGI_TRY_HIP(hipMemcpyAsync(b->dev[a], b->host[a], b->arena_bytes, hipMemcpyHostToDevice, lanes.main));
+    VGI_TRY_HIP(hipMemcpyAsync(b->dev[a], b->host[a], b->split ? b->arena_bytes : b->unsplit_bytes, hipMemcpyHostToDevice,
+                               lanes.main));
     for (int s = 0; s < kSlotCount; ++s) {
         const int kind = slot_kind(s);
         const BatchOps* o = batch_ops(kind);
         const BatchHeader* hd = (const BatchHeader*)((const char*)b->host[a] + b->offsets[s]);
         if (!all_slots && hd->njobs == 0) continue;
+        if (all_slots && (s == kSlotTimedSpec || s == kSlotTimedDiff)) continue;  // never used in a graph
         hipStream_t st;
         vgi_status r = lanes.enter(s, st);
         if (r != VGI_OK) return r;
         if (profile) {
-            ProfScope prof(kind_name(kind), st, 0.0);
+            const uint32_t part = b->split ? split_part(s) : (uint32_t)kSamplePassCount;
+            ProfScope prof(part == kSamplePassCount ? kind_name(kind) : sample_pass_name(part, true), st, 0.0);
             r = o->launch((const char*)b->dev[a] + b->offsets[s], storage, groups_for(b, s, o), o->trace ? lds : 0, st);
         } else {
             r = o->launch((const char*)b->dev[a] + b->offsets[s], storage, groups_for(b, s, o), o->trace ? lds : 0, st);
@@ -236,10 +282,9 @@ extern "C" vgi_status vgi_batch_add_passes(vgi_batch* b, const vgi_scene* scene,
     const int a = b->flip;
     if (b->used[a]) VGI_TRY_HIP(hipEventSynchronize(b->done[a]));
     const PassRec* list[kMaxBatchViews];
+    b->split = !b->cfg.use_graph && timing_sample_passes(true);
     for (int s = 0; s < kSlotCount; ++s) {
-        int n = 0;
-        for (uint32_t v = 0; v < num_views; ++v)
-            if (b->recs[v].has[s]) list[n++] = &b->recs[v].recs[s];
+        const int n = slot_records(b, s, num_views, list);
         const BatchOps* o = batch_ops(slot_kind(s));
         vgi_status r = o->fill(list, n, (char*)b->host[a] + b->offsets[s]);
         if (r != VGI_OK) return r;

@@ -62,7 +62,9 @@ enum Slot : int {
     kSlotHgRaygen,
     kSlotHgRaygenOrdered,
     kSlotSampleSpec,  // issued ahead of the diffuse passes
+    kSlotTimedSpec,   // second half of a lobe whose passes a batch launches apart to time them
     kSlotSampleDiff,
+    kSlotTimedDiff,
     kSlotAoGen,
     kSlotAoFilter,
     kSlotDiffTemporal,
@@ -88,7 +90,8 @@ inline int slot_kind(int slot) {
         kPassGBuffer,      kPassClear,        kPassClear,         kPassClear,       kPassClear,       kPassHgDecay,
         kPassClear,        kPassHgSelect,     kPassClear,         kPassHgSelectOrdered, kPassClear, kPassHgCompact,
         kPassHgCompactOrdered, kPassClear,    kPassHgRaygen,      kPassHgRaygenOrdered,
-        kPassSampleSpec,   kPassSampleDiff,   kPassAoGen,        kPassAoFilter,      kPassDiffTemporal, kPassDiffSpatial, kPassSpecTemporal,
+        kPassSampleSpec,   kPassSampleSpec,   kPassSampleDiff,   kPassSampleDiff,    kPassAoGen,        kPassAoFilter,
+        kPassDiffTemporal, kPassDiffSpatial,  kPassSpecTemporal,
         kPassSpecSpatial,  kPassClear,        kPassClear,         kPassDenTemporal, kPassDenDisocclusion,
         kPassDenFastClamp, kPassDenFallback,  kPassDenAtrous,     kPassDenAtrous,   kPassDenAtrous,
         kPassDenAtrous,    kPassDenAtrous,    kPassShadow,        kPassFinalLighting, kPassTemporalAA};
@@ -109,6 +112,14 @@ struct SampleSet {
     vgi_ind_spec_sample_gen_io spec_gen;
     vgi_pc_sample_gen diff_pc, spec_pc;
     void add(SamplePass p) { pass[count++] = p; }
+    // Keeps pass `p` only; whether it was there.
+    bool keep(SamplePass p) {
+        bool has = false;
+        for (uint32_t k = 0; k < count; ++k) has |= pass[k] == p;
+        count = has ? 1u : 0u;
+        pass[0] = p;
+        return has;
+    }
     bool spec() const { return pass[0] == kSampleSpecValidate || pass[0] == kSampleSpecGen; }
 };
 
@@ -209,7 +220,7 @@ inline int slot_phase(int slot) {
     return slot < kSlotSampleSpec ? 0 : slot < kSlotDenClearFastDiff ? 1 : slot < kSlotFinalLighting ? 2 : 3;
 }
 inline int slot_lane(int slot) {
-    return (slot >= kSlotClearHgStorage && slot <= kSlotSampleSpec) || slot == kSlotSpecTemporal ||
+    return (slot >= kSlotClearHgStorage && slot <= kSlotTimedSpec) || slot == kSlotSpecTemporal ||
            slot == kSlotSpecSpatial || slot == kSlotShadow;
 }
 
@@ -253,6 +264,10 @@ vgi_status launch_compact_ordered_fresh(const vgi_hash_grid_ordered_compact_io* 
                                         hipStream_t st);
 // The launch of a kPassSampleSpec or kPassSampleDiff record (vgi_sample.hip).
 vgi_status launch_sample_rays(const PassRec& r, hipStream_t st);
+// A sample pass's name in the profiler (`batch`: of a batch's launches), and
+// whether the timers ask for one of the four.
+const char* sample_pass_name(uint32_t pass, bool batch);
+bool timing_sample_passes(bool batch);
 
 // Keeps the records of one view's frame by slot.
 struct RecordSink : PassSink {

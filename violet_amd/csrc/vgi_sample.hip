@@ -457,13 +457,16 @@ struct BatchMinWaves<JobSpecRays<S>> {
     static constexpr int value = kTraceWaves;
 };
 
-static const char* sample_pass_name(uint32_t pass) {
-    switch (pass) {
-        case kSampleSpecValidate: return "ind_spec_sample_validate";
-        case kSampleDiffGen: return "ind_diff_sample_gen";
-        case kSampleDiffValidate: return "ind_diff_sample_validate";
-        default: return "ind_spec_sample_gen";
-    }
+const char* sample_pass_name(uint32_t pass, bool batch) {
+    static const char* n[kSamplePassCount] = {"batch_ind_spec_sample_validate", "batch_ind_diff_sample_gen",
+                                              "batch_ind_diff_sample_validate", "batch_ind_spec_sample_gen"};
+    return n[pass] + (batch ? 0 : 6);
+}
+
+bool timing_sample_passes(bool batch) {
+    for (uint32_t k = 0; k < kSamplePassCount; ++k)
+        if (profiling_pass(sample_pass_name(k, batch))) return true;
+    return false;
 }
 
 // What the entry points of the single passes check, for each pass of a set;
@@ -506,7 +509,7 @@ static vgi_status check_sample_set(const vgi_trace_resources* tr, const SampleSe
                 break;
             }
         }
-        const char* name = sample_pass_name(a.pass[k]);
+        const char* name = sample_pass_name(a.pass[k], false);
         VGI_REQUIRE(valid_dims(pw, ph), "vgi_pass_%s: bad size", name);
         VGI_REQUIRE(storage == tr->storage, "vgi_pass_%s: storage mismatch", name);
         VGI_REQUIRE(bound, "vgi_pass_%s: missing binding", name);
@@ -616,8 +619,7 @@ namespace vgi {
 vgi_status launch_sample_rays(const PassRec& r, hipStream_t st) {
     const SampleSet& a = r.io.sample;
     void* s = (void*)st;
-    if (!trace_counters() && !profiling_pass("ind_diff_sample_gen") && !profiling_pass("ind_diff_sample_validate") &&
-        !profiling_pass("ind_spec_sample_gen") && !profiling_pass("ind_spec_sample_validate"))
+    if (!trace_counters() && !timing_sample_passes(false))
         return launch_sample_set(a.spec() ? "ind_spec_sample" : "ind_diff_sample", 0.0, &r.fp, &r.tr, a, st);
     for (uint32_t k = 0; k < a.count; ++k) switch (a.pass[k]) {
             case kSampleSpecValidate: VGI_CHECK(vgi_pass_ind_spec_sample_validate(&r.fp, &r.tr, &a.spec_validate, s)); break;

@@ -24,6 +24,12 @@ frame fence (crates/violet-app/src/render_loop.rs:445-482), a batch still
 running `frame_timeout_ms` after its issue is counted as timed out and
 waited for further, and one finishing after 33.3 ms as slow.
 
+`on_complete(request, view, outputs)` is called when a request's batch has
+finished.  The outputs are the view's own images, which its next frame writes
+again: device work that the callback issues on the current stream (a copy of
+them) is ordered before that frame; work on another stream has to be waited
+for before the callback returns.
+
 Metrics: with `metrics` (a path or an open text file) the server appends
 one JSON line per completed batch (slot, issue time, batch time, views,
 pixels, each request's latency, whether it timed out) and a summary line
@@ -123,6 +129,7 @@ class Server:
         self.frame_of: dict[int, int] = collections.defaultdict(int)
         self.last_use: dict[int, float] = {}
         self.inflight_views: set[int] = set()
+        self.reads: dict[int, "torch.cuda.Event"] = {}  # per view: after what on_complete issued for it
         self.bytes_resident = 0
         self.view_bytes: dict[int, int] = {}
         # device bytes of a view are affine in its pixel count: measure the
@@ -191,6 +198,9 @@ class Server:
                 self.last_use[req.view] = t_done
                 if self.on_complete:
                     self.on_complete(req, self.resident[req.view], outs)
+                    ev = self.torch.cuda.Event()
+                    ev.record(self.torch.cuda.current_stream())
+                    self.reads[req.view] = ev
             self.busy[k] = None
 
     def _issue(self, k: int, queue: collections.deque, now: float, stats: ServeStats) -> None:
@@ -215,6 +225,10 @@ class Server:
         rs = [self.resident[r.view] for r in picked]
         fps = [view_frame_params(self.views[r.view], self.frame_of[r.view]) for r in picked]
         idx = [self.frame_of[r.view] for r in picked]
+        for r in picked:
+            ev = self.reads.pop(r.view, None)
+            if ev is not None:
+                stream.wait_event(ev)
         with self.torch.cuda.stream(stream):
             outs = bt.add_passes(self.scene, rs, fps, idx, stream=stream.cuda_stream)
             self.fences[k].record(stream.cuda_stream)

@@ -1,10 +1,10 @@
 // Host-code fuzz driver for the sanitizer builds (AddressSanitizer and
-// UndefinedBehaviorSanitizer): the glTF importer (vgi_gltf.cpp) on every
-// document named on the command line, and the scene builder (the host half of
-// vgi_scene_create: validation, binned SAH, 4-wide collapse, quantised nodes)
-// on each imported model and on seeded triangle soups, some of them invalid.
-// Nothing here touches a GPU.  Exit status 0 unless an invariant fails; a
-// sanitizer report aborts the process.
+// UndefinedBehaviorSanitizer; ThreadSanitizer without documents): the glTF
+// importer (vgi_gltf.cpp) on every document named on the command line, and the
+// scene builder (the host half of vgi_scene_create: validation, binned SAH,
+// 4-wide collapse, quantised nodes) on each imported model and on seeded
+// triangle soups, some of them invalid.  Nothing here touches a GPU.  Exit
+// status 0 unless an invariant fails; a sanitizer report aborts the process.
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -87,9 +87,11 @@ int main(int argc, char** argv) {
         }
         vgi_gltf_destroy(m);
     }
-    // triangle soups: clustered, degenerate, huge, non-finite, bad indices
-    for (int s = 0; s < 60; ++s) {
-        const uint32_t nt = 1 + next() % (s < 50 ? 3000u : 20u), nv = 3 * nt;
+    // triangle soups: clustered, degenerate, huge, non-finite, bad indices; the
+    // last ones large enough that the builder builds subtrees on threads
+    uint64_t hash = 1469598103934665603ull;  // FNV-1a of every built tree
+    for (int s = 0; s < 66; ++s) {
+        const uint32_t nt = s >= 60 ? 40000u : 1 + next() % (s < 50 ? 3000u : 20u), nv = 3 * nt;
         std::vector<float> pos(3 * (size_t)nv), nrm(3 * (size_t)nv, 0.0f);
         std::vector<uint32_t> idx(3 * (size_t)nt), tm(nt, 0);
         const int kind = s % 6;
@@ -123,9 +125,11 @@ int main(int argc, char** argv) {
         if (st == VGI_OK) {
             ++built;
             check_scene(hs, nt, "soup");
+            for (const BvhNode& n : hs.nodes)
+                for (size_t k = 0; k < sizeof(n); ++k) hash = (hash ^ ((const unsigned char*)&n)[k]) * 1099511628211ull;
         }
     }
-    std::printf("host_fuzz: %d documents (%d imported), %d scenes (%d built), %d failures\n", docs, imported, scenes,
-                built, failures);
+    std::printf("host_fuzz: %d documents (%d imported), %d scenes (%d built), %d failures, trees %016llx\n", docs,
+                imported, scenes, built, failures, (unsigned long long)hash);
     return failures ? 1 : 0;
 }

@@ -8,8 +8,11 @@ sanitizers).
   `sanitize/host_fuzz.cpp` on the corrupted-document corpus of the import
   fuzz test (untextured, PNG- and JPEG-textured documents), the reference's own glTF
   assets when present, and seeded triangle soups (clustered, degenerate,
-  huge, non-finite, bad indices).
+  huge, non-finite, bad indices), some of 40,000 triangles, whose subtrees
+  build on threads.
   Every built scene is checked: each triangle in exactly one leaf.
+* ThreadSanitizer (gcc) on the scene builder with the same soups; the trees
+  are the same on one processor as on all.
 * ThreadSanitizer on the oracle's OpenMP twin (clang with LLVM's OpenMP
   runtime and its Archer tool, which tells ThreadSanitizer about OpenMP's
   synchronisation): `sanitize/oracle_race.c` runs two frames of the G-buffer,
@@ -38,6 +41,33 @@ def _run(cmd, env=None, timeout=600):
     return r.returncode, r.stdout + r.stderr
 
 
+def _host_fuzz(tmp_path, sanitizers):
+    csrc = ROOT / "violet_amd" / "csrc"
+    exe = tmp_path / "host_fuzz"
+    cmd = ["g++", "-std=c++17", "-O1", "-g", "-fno-omit-frame-pointer", f"-fsanitize={sanitizers}",
+           "-fno-sanitize-recover=all", "-pthread", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM / 'include'}",
+           f"-I{ROOT / 'include'}", f"-I{csrc}", str(HERE / "sanitize" / "host_fuzz.cpp"), str(csrc / "vgi_gltf.cpp"),
+           str(csrc / "vgi_bvh.cpp"), str(csrc / "vgi_image.cpp"), str(csrc / "vgi_runtime.cpp"), f"-L{ROCM / 'lib'}",
+           "-lamdhip64", f"-Wl,-rpath,{ROCM / 'lib'}", "-o", str(exe)]
+    rc, out = _run(cmd)
+    assert rc == 0, out[-4000:]
+    return exe
+
+
+@pytest.mark.skipif(shutil.which("g++") is None or not (ROCM / "include" / "hip").exists(),
+                    reason="needs g++ and the HIP headers")
+def test_scene_builder_threads_under_thread_sanitizer(tmp_path):
+    exe = _host_fuzz(tmp_path, "thread")
+    env = dict(os.environ, TSAN_OPTIONS="halt_on_error=1 exitcode=66 ignore_noninstrumented_modules=1")
+    rc, out = _run([str(exe)], env=env)
+    assert rc == 0 and "WARNING: ThreadSanitizer" not in out and "0 failures" in out, out[-4000:]
+    cpus = os.sched_getaffinity(0)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, env=env, timeout=600,
+                       preexec_fn=lambda: os.sched_setaffinity(0, {min(cpus)}))
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert out.split("trees ")[1] == r.stdout.split("trees ")[1]
+
+
 @pytest.mark.skipif(shutil.which("g++") is None or not (ROCM / "include" / "hip").exists(),
                     reason="needs g++ and the HIP headers")
 def test_host_code_under_address_and_undefined_behaviour_sanitizers(tmp_path):
@@ -45,15 +75,7 @@ def test_host_code_under_address_and_undefined_behaviour_sanitizers(tmp_path):
     from restir_harness import make_mesh
     from test_gltf_import import _build
 
-    csrc = ROOT / "violet_amd" / "csrc"
-    exe = tmp_path / "host_fuzz"
-    cmd = ["g++", "-std=c++17", "-O1", "-g", "-fno-omit-frame-pointer", "-fsanitize=address,undefined",
-           "-fno-sanitize-recover=all", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM / 'include'}", f"-I{ROOT / 'include'}",
-           f"-I{csrc}", str(HERE / "sanitize" / "host_fuzz.cpp"), str(csrc / "vgi_gltf.cpp"), str(csrc / "vgi_bvh.cpp"),
-           str(csrc / "vgi_image.cpp"),
-           str(csrc / "vgi_runtime.cpp"), f"-L{ROCM / 'lib'}", "-lamdhip64", f"-Wl,-rpath,{ROCM / 'lib'}", "-o", str(exe)]
-    rc, out = _run(cmd)
-    assert rc == 0, out[-4000:]
+    exe = _host_fuzz(tmp_path, "address,undefined")
     docs = corrupted_documents(_build()[0], tmp_path / "a", seed=99)
     docs += corrupted_documents(scene_from_mesh(make_mesh(300)), tmp_path / "b", seed=7)
     # textured: PNG images (decoding, mips) and texture slots in the damaged files

@@ -7,10 +7,10 @@
  * renderer's own sequencer into per-slot records, writes one table per slot
  * into a pinned host arena, uploads the arena with a single copy and runs
  * every slot as one persistent launch over all views (vgi_batch.h).  The
- * launch shapes depend only on the batch configuration, the storage mode
- * and the scene's traversal-stack size, so the whole frame can be captured
- * once as a HIP graph and replayed; the tables it reads are the only
- * per-frame input.  Two arenas alternate so the host can fill one while the
+ * launch shapes depend only on the batch configuration, the storage mode,
+ * the vgi_tuning shapes and the largest tile counts seen, so the whole frame
+ * can be captured once as a HIP graph and replayed until one of these
+ * changes; the tables it reads are the only per-frame input.  Two arenas alternate so the host can fill one while the
  * device still reads the other.
  */
 #include <new>
@@ -74,7 +74,6 @@ struct vgi_batch {
     hipGraphExec_t exec[2] = {nullptr, nullptr};
     uint32_t key_storage[2] = {0, 0};
     uint32_t key_shape[2][2] = {{0, 0}, {0, 0}};  // launch shapes (vgi_tuning) the graph was captured with
-    size_t key_lds[2] = {0, 0};
     // One-group-per-tile slots launch as many groups as the largest tile
     // count seen so far for the slot (a graph is re-captured when it grows).
     uint32_t grid_bound[kSlotCount];
@@ -300,7 +299,7 @@ extern "C" vgi_status vgi_batch_add_passes(vgi_batch* b, const vgi_scene* scene,
         VGI_TRY_HIP(hipEventRecord(b->done[a], st));
     } else {
         const uint32_t shape[2] = {tuning_atrous_block(), tuning_trace_tile_width()};
-        if (!b->exec[a] || b->key_storage[a] != storage || b->key_lds[a] != lds ||
+        if (!b->exec[a] || b->key_storage[a] != storage ||
             memcmp(b->key_grid[a], b->grid_bound, sizeof(b->grid_bound)) != 0 ||
             memcmp(b->key_shape[a], shape, sizeof(shape)) != 0) {
             if (b->exec[a]) {
@@ -320,7 +319,6 @@ extern "C" vgi_status vgi_batch_add_passes(vgi_batch* b, const vgi_scene* scene,
             (void)hipGraphDestroy(g);
             VGI_TRY_HIP(e);
             b->key_storage[a] = storage;
-            b->key_lds[a] = lds;
             memcpy(b->key_grid[a], b->grid_bound, sizeof(b->grid_bound));
             memcpy(b->key_shape[a], shape, sizeof(shape));
         }

@@ -411,8 +411,8 @@ static FrameParams to_fp(const vgi_frame_params* fp) {
     } while (0)
 
 // ---------------------------------------------------------------------------
-// Fused multi-view launches (vgi_batch.h); the scene (and so the LDS stack
-// size) is shared by every view of a batch.
+// Fused multi-view launches (vgi_batch.h); the scene is shared by every view
+// of a batch.
 // ---------------------------------------------------------------------------
 template <class S, bool kSpec>
 struct JobSampleRays {

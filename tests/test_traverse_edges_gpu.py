@@ -43,14 +43,20 @@ def _check(vgi, mesh, rays):
 @pytest.mark.parametrize("interval", [(5e-4, 1000.0), (-3.0, 1000.0), (0.0, np.inf), (0.5, 1.5)])
 def test_edges(vgi, n_tris, copies, n_rays, interval):
     rng = np.random.default_rng(n_tris + n_rays)
+    mesh = _soup(n_tris, 3, copies)
     o = rng.uniform(-2.0, 2.0, (n_rays, 3))
     d = rng.uniform(-1.0, 1.0, (n_rays, 3)) - o
+    # every other ray from one unit off a triangle's middle, about along its normal: a sure hit in all intervals
+    aimed = np.arange(n_rays) % 2 == 0
+    tri = mesh.positions[mesh.indices[rng.integers(0, len(mesh.indices), n_rays)]].astype(np.float64)
+    normal = np.cross(tri[:, 1] - tri[:, 0], tri[:, 2] - tri[:, 0])
+    normal /= np.linalg.norm(normal, axis=1, keepdims=True)
+    d[aimed] = (normal * rng.choice([-1, 1], (n_rays, 1)) + rng.uniform(-0.3, 0.3, (n_rays, 3)))[aimed]
     d /= np.linalg.norm(d, axis=1, keepdims=True)
+    o[aimed] = (tri.mean(1) - d)[aimed]
     one = np.ones((n_rays, 1))
     rays = np.concatenate([o, interval[0] * one, d, interval[1] * one], 1).astype(np.float32)
-    hit = _check(vgi, _soup(n_tris, 3, copies), rays)
-    if n_tris == 300 and n_rays == 1000:
-        assert hit.any()
+    assert _check(vgi, mesh, rays)[aimed].all()
 
 
 def test_stack_leaves_lds_twice(vgi):

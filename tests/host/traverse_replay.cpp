@@ -10,8 +10,8 @@
 // Prints: rays, hits, lost (closest hit differs), any (any-hit answer differs),
 // the most stack entries of a lane, the most moves to private memory of a lane,
 // node steps of all waves, how many of them did stack moves, how many had a
-// lane with entries to move, and the lanes that sat out a node step because all
-// they had left was in private memory.
+// lane with entries to move, and the node steps with all of every stack in LDS.
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -61,8 +61,7 @@ bool closer_hit(f3 o, f3 d, const BvhTri& tr, float tmin, RayHit& h) {
 struct Totals {
     long long steps = 0, move_steps = 0, needed_steps = 0;
     int max_entries = 0, max_moves = 0;
-    long long idle = 0;
-} totals;
+};
 
 struct Lane {
     bool used = false;
@@ -72,18 +71,15 @@ struct Lane {
     RayHit h;
     int32_t node, leaf = 0;
     uint32_t base, p;
-    int32_t lds[kLdsStackEntries];
+    std::vector<int32_t> lds;
     int32_t spill[kStackMaxEntries];
     int spilled = 0, moves = 0;
     int32_t& at(uint32_t a) {
         const uint32_t off = a - base;
-        require(off % kStackStride == 0 && off / kStackStride < kLdsStackEntries, "LDS stack access out of range");
+        require(off % kStackStride == 0 && off / kStackStride < lds.size(), "LDS stack access out of range");
         return lds[off / kStackStride];
     }
-    void entries() {
-        const int n = (int32_t)(p - base) / (int32_t)kStackStride + spilled;
-        if (n > totals.max_entries) totals.max_entries = n;
-    }
+    int entries() const { return (int32_t)(p - base) / (int32_t)kStackStride + spilled; }
 };
 
 float safe_dir(float v) { return std::fabs(v) < 1e-20f ? std::copysign(1e-20f, v) : v; }
@@ -109,9 +105,11 @@ bool slab(const Lane& l, const BvhNode& n, int k, float& tn) {
 // Nothing left but entries in private memory.
 bool waits(const Lane& l) { return l.used && l.spilled > 0 && l.node == kDone && l.leaf == 0; }
 
+// `bounded`: with the stack in two parts; else all of it in "LDS".
 template <bool kAny>
-void run_wave(const HostScene& s, std::vector<Lane>& w) {
+void run_wave(const HostScene& s, std::vector<Lane>& w, Totals& totals, bool bounded = true) {
     for (Lane& l : w) {
+        l.lds.assign(bounded ? kLdsStackEntries : kStackMaxEntries + 8, 0);
         l.p = l.base;
         l.at(l.p) = kDone;
         l.at(l.p + kStackStride) = kDone;
@@ -119,19 +117,6 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
     }
     bool deep = false;
     for (;;) {
-        if (deep)
-            for (Lane& l : w)
-                if (waits(l)) {
-                    l.spilled -= kSpillEntries;
-                    for (int k = 0; k < kSpillEntries; ++k) l.at(l.base + kStackStride * (2 + k)) = l.spill[l.spilled + k];
-                    l.p = l.base + kStackStride * (kSpillEntries - 1);
-                    l.node = l.at(l.p + 2 * kStackStride);
-                    if (is_leaf(l.node)) {
-                        l.leaf = l.node;
-                        l.node = l.at(l.p + kStackStride);
-                        l.p -= kStackStride;
-                    }
-                }
         int n_leaf = 0, n_want = 0;
         for (const Lane& l : w) {
             if (!l.used) continue;
@@ -145,16 +130,15 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
             for (size_t k = 0; k < w.size(); ++k) {
                 const Lane& l = w[k];
                 if (!l.used) continue;
-                totals.idle += waits(l);
                 inner |= (uint64_t)(l.node >= 0) << k;
-                over |= (uint64_t)stack_over(l.p, l.base) << k;
-                need |= l.node >= 0 && (int32_t)(l.p - l.base) > (int32_t)(kStackStride * (kLdsStackEntries - 6));
+                over |= (uint64_t)(bounded && stack_over(l.p, l.base)) << k;
+                need |= bounded && l.node >= 0 && (int32_t)(l.p - l.base) > (int32_t)(kStackStride * (kLdsStackEntries - 6));
             }
             totals.move_steps += full_stacks(inner, over) != 0;
             totals.needed_steps += need;
             for (Lane& l : w) {
                 if (!l.used || l.node < 0) continue;
-                if (stack_over(l.p, l.base)) {
+                if (bounded && stack_over(l.p, l.base)) {
                     require(l.spilled + kSpillEntries <= (int)kStackMaxEntries, "private stack full");
                     for (int k = 0; k < kSpillEntries; ++k) l.spill[l.spilled + k] = l.at(l.base + kStackStride * (2 + k));
                     l.spilled += kSpillEntries;
@@ -189,14 +173,17 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
                     for (int k = 0; k < 4; ++k) l.at(l.p + (2 + k) * kStackStride) = n.link[order[k]];
                     l.p += kStackStride * cnt;
                 }
-                l.entries();
+                totals.max_entries = std::max(totals.max_entries, l.entries());
                 const int32_t e0 = l.at(l.p + kStackStride), e1 = l.at(l.p);
                 const bool aside = l.leaf == 0 && is_leaf(e0);
                 l.leaf = aside ? e0 : l.leaf;
                 l.node = aside ? e1 : e0;
                 l.p -= aside ? 2 * kStackStride : kStackStride;
             }
-        } else if (n_leaf != 0) {
+        } else {
+            bool left = n_leaf != 0;
+            for (const Lane& l : w) left |= l.used && l.spilled > 0;
+            if (!left) break;
             for (Lane& l : w) {
                 if (!l.used || l.leaf == 0) continue;
                 const uint32_t enc = ~(uint32_t)l.leaf, first = enc >> 4, n = enc & 15u;
@@ -213,8 +200,19 @@ void run_wave(const HostScene& s, std::vector<Lane>& w) {
                     l.p -= kStackStride;
                 }
             }
-        } else {
-            break;
+            if (deep)
+                for (Lane& l : w)
+                    if (waits(l)) {
+                        l.spilled -= kSpillEntries;
+                        for (int k = 0; k < kSpillEntries; ++k) l.at(l.base + kStackStride * (2 + k)) = l.spill[l.spilled + k];
+                        l.p = l.base + kStackStride * (kSpillEntries - 1);
+                        l.node = l.at(l.p + 2 * kStackStride);
+                        if (is_leaf(l.node)) {
+                            l.leaf = l.node;
+                            l.node = l.at(l.p + kStackStride);
+                            l.p -= kStackStride;
+                        }
+                    }
         }
     }
     for (const Lane& l : w) require(!l.used || l.spilled == 0, "a lane ended with entries in private memory");
@@ -249,6 +247,7 @@ int main(int argc, char** argv) {
     HostScene s;
     require(build_scene_host(&desc, s) == VGI_OK, "scene refused");
 
+    Totals totals, unbounded;
     long long hits = 0, lost = 0, any = 0;
     for (uint32_t r0 = 0; r0 < n[2]; r0 += 64) {
         std::vector<Lane> w(64);
@@ -273,9 +272,12 @@ int main(int argc, char** argv) {
             if (w[k].used)
                 for (const BvhTri& t : s.tris) closer_hit(w[k].o, w[k].d, t, w[k].tmin, brute[k]);
         }
-        std::vector<Lane> wa = w;
-        run_wave<false>(s, w);
-        run_wave<true>(s, wa);
+        const std::vector<Lane> start = w;
+        std::vector<Lane> wa = w, whole = w;
+        run_wave<false>(s, w, totals);
+        run_wave<true>(s, wa, totals);
+        run_wave<false>(s, whole, unbounded, false);
+        run_wave<true>(s, whole = start, unbounded, false);
         for (int k = 0; k < 64; ++k) {
             if (!w[k].used) continue;
             const bool hit = brute[k].tri != 0xFFFFFFFFu;
@@ -285,8 +287,8 @@ int main(int argc, char** argv) {
         }
     }
     std::printf("rays %u hits %lld lost %lld any %lld max_entries %d max_moves %d steps %lld move_steps %lld "
-                "needed_steps %lld idle %lld nodes %zu\n",
+                "needed_steps %lld unbounded_steps %lld nodes %zu\n",
                 n[2], hits, lost, any, totals.max_entries, totals.max_moves, totals.steps, totals.move_steps,
-                totals.needed_steps, totals.idle, s.nodes.size());
+                totals.needed_steps, unbounded.steps, s.nodes.size());
     return 0;
 }

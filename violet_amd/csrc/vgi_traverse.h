@@ -210,12 +210,13 @@ __device__ __forceinline__ bool closer_hit(f3 o, f3 d, Vf4 v0, Vf4 e1v, Vf4 e2v,
 // hits do not depend on the visiting order (closest t, then lowest id), only
 // the work does.
 //
-// A lane whose LDS part is empty takes back what it moved to private memory at
-// once.  Leaving that until no lane of the wave had anything else to do made
-// deep rays finish alone: 256 rays from inside a pile of 200,000 quads 451 ->
-// 216 us, a million 2620 -> 2263 us, a million slanted ones 418 -> 391 us.  It
-// had also kept in step waves whose halves cross the pile in opposite
-// directions: those 292 -> 369 us.
+// A lane whose LDS part is empty takes back what it moved to private memory
+// after the wave's next leaf step.  Leaving that until no lane of the wave had
+// anything else to do made deep rays finish alone: 256 rays from inside a pile
+// of 200,000 quads 447 -> 207 us, a million 2627 -> 2255 us.  It had also kept
+// in step waves whose halves cross the pile in opposite directions: those 298
+// -> 367 us.  A look at every node step instead costs small frames 0.4%.
+// Any-hit rays end early and gain nothing by it (33 -> 31 us); they wait.
 //
 // 1M bounce rays on 1M triangles: 324 -> 241 us; the 1080p sampling and
 // spatial passes 1210 -> 995 us; a 1080p frame 1951 -> 1687 us, a 256x256 one
@@ -244,33 +245,33 @@ __device__ __forceinline__ Hit traverse(const SceneView& s, f3 o, f3 d, float tm
     static_assert(kStackStride == 256u, "the offsets below");
     int32_t spill[kStackMaxEntries];
     int32_t spilled = 0;
+    auto take_back = [&]() {
+        if (spilled > 0 && node == kTraversalDone && leaf == 0) {
+            spilled -= kSpillEntries;
+            for (int k = 0; k < kSpillEntries; ++k) lds_at(base + 256u * (2 + k)) = spill[spilled + k];
+            p = base + 256u * (kSpillEntries - 1);
+            node = lds_at(p + 512u);
+            if (is_leaf(node)) {
+                leaf = node;
+                node = lds_at(p + 256u);
+                p -= 256u;
+            }
+        }
+    };
     // Every step of the wave moves at least one lane, and each node and leaf
     // of a tree is reached at most once per lane (a node has at most 4
     // children); the budget only guards against a corrupted BVH turning into
     // an endless loop.
     uint32_t budget = s.num_nodes < (1u << 23) ? 64u * (5u * s.num_nodes + 8u) : 0xFFFFFFFFu;
-    bool live = true;
-    bool deep = false;  // a lane of the wave has moved entries to private memory
-    while (live) {
-        if (deep) {
-            if (spilled > 0 && node == kTraversalDone && leaf == 0) {
-                spilled -= kSpillEntries;
-                for (int k = 0; k < kSpillEntries; ++k) lds_at(base + 256u * (2 + k)) = spill[spilled + k];
-                p = base + 256u * (kSpillEntries - 1);
-                node = lds_at(p + 512u);
-                if (is_leaf(node)) {
-                    leaf = node;
-                    node = lds_at(p + 256u);
-                    p -= 256u;
-                }
-            }
-        }
+    uint64_t m_deep = 0;  // lanes that have moved entries to private memory
+    for (;;) {
         const bool inner = node >= 0;
         const uint64_t m_inner = __ballot(inner), m_leaf = __ballot(leaf != 0);
         const uint64_t m_want = m_inner & ~m_leaf;
         if (m_want != 0 && 3 * (int)__popcll(m_want) >= 2 * (int)__popcll(m_leaf)) {
-            if (full_stacks(m_inner, __ballot(stack_over(p, base))) != 0) {  // rare
-                deep = true;
+            const uint64_t m_full = full_stacks(m_inner, __ballot(stack_over(p, base)));
+            m_deep |= m_full;
+            if (m_full != 0) {  // rare
                 if (inner && stack_over(p, base)) {
                     if (spilled + kSpillEntries <= (int32_t)kStackMaxEntries) {
                         for (int k = 0; k < kSpillEntries; ++k) spill[spilled + k] = lds_at(base + 256u * (2 + k));
@@ -369,11 +370,13 @@ __device__ __forceinline__ Hit traverse(const SceneView& s, f3 o, f3 d, float tm
                     p -= 256u;
                 }
             }
+            if (!kAnyHit && m_deep != 0) take_back();
         } else {
-            live = false;  // every lane's stack is empty
+            if (__ballot(spilled > 0) == 0) break;  // every lane's stack is empty
+            take_back();
         }
         budget = __builtin_amdgcn_readfirstlane(budget) - 1u;
-        live = live && budget != 0u;
+        if (budget == 0u) break;
     }
     if (kCount) count_traversal(s, kAnyHit, n_nodes, n_tris);
     return h;

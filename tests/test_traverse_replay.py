@@ -50,10 +50,11 @@ def replay(tmp_path_factory):
     return run
 
 
-def mixed_scale(width, far, axis, n_rays, seed):
+def mixed_scale(width, far, axis, n_rays, seed, away=0.0):
     """A square of 16 x 16 tiles of edge width / 16 across `axis` through the
     origin, one triangle about `far` units away, and rays at the square from
-    within two widths of it: grazing it, or across it along the axes."""
+    within two widths of it (`away` further back): grazing it, or across it
+    along the axes."""
     rng = np.random.default_rng(seed)
     n = 16
     g = np.linspace(-width / 2, width / 2, n + 1)
@@ -71,9 +72,9 @@ def mixed_scale(width, far, axis, n_rays, seed):
     k = n_rays // 8  # straight down onto the square, at tile borders too
     d[:k] = [0, 0, 1]
     target[: k // 2, 0] = rng.choice(g, k // 2)
-    o = target - d * (2 * width * rng.uniform(0.2, 1.0, (n_rays, 1)))
+    o = target - d * (away + 2 * width * rng.uniform(0.2, 1.0, (n_rays, 1)))
     one = np.ones((n_rays, 1))
-    rays = np.concatenate([np.roll(o, axis, 1), 5e-4 * one, np.roll(d, axis, 1), 1000.0 * one], 1)
+    rays = np.concatenate([np.roll(o, axis, 1), 5e-4 * one, np.roll(d, axis, 1), (1000.0 + 2 * away) * one], 1)
     return np.roll(pos, axis, 1).astype(np.float32), idx.astype(np.uint32), rays.astype(np.float32)
 
 
@@ -81,6 +82,15 @@ def mixed_scale(width, far, axis, n_rays, seed):
 @pytest.mark.parametrize("width,far", [(1.0, -900.0), (1.0, 300.0), (4.0, -4000.0)])
 def test_mixed_scales_lose_no_hit(replay, width, far, axis):
     r = replay(*mixed_scale(width, far, axis, 60000, seed=2))
+    assert r["hits"] > 0.99 * r["rays"]
+    assert r["lost"] == 0 and r["any"] == 0, r
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_a_thousand_units_away(replay, axis):
+    """Rays from far outside, whose errors go with their distance: the outermost planes of a node have
+    room for them."""
+    r = replay(*mixed_scale(1.0, -900.0, axis, 100000, seed=axis, away=1000.0))
     assert r["hits"] > 0.99 * r["rays"]
     assert r["lost"] == 0 and r["any"] == 0, r
 

@@ -299,6 +299,7 @@ int32_t build_tree(Builder& b, int n, Box& root_box) {
 // leaf its area times its triangles.
 struct Collapser {
     const std::vector<Node2>& n2;
+    float reach;  // the scene's largest coordinate magnitude
     std::vector<BvhNode> out;
     int max_level = 0;
     struct Cost {
@@ -390,14 +391,20 @@ struct Collapser {
     // from its box widened by m, so its grid box keeps at least m between
     // itself and the padded box (the divisions are in double, and the loops
     // after them settle a quotient that rounding moved across a whole number).
-    // m covers what the traversal's plane distances err by on the scale of the
-    // node (slab_q: 2^-23 of its extent and 3 * 2^-24 of its origin), which
-    // the padding cannot: it goes with the child's own coordinates.  Without
-    // it, rays grazing a unit-sized floor whose node also held a triangle 900
-    // units away lost 104 of 100,000 hits.  On the scene of a million
-    // triangles rays visit as many nodes with it as without (camera rays
-    // 13.053, bounce rays 22.710 against 22.709, shadow rays 13.668).
-    static void quantise(BvhNode& nd, const Box* box, const int32_t* child, int cnt) {
+    // m covers the rounding of the traversal's plane distances (slab_q), which
+    // the padding cannot, as that goes with the child's own coordinates:
+    // - on the scale of the node, 2^-23 of its extent and 3 * 2^-24 of its
+    //   origin.  Without it, rays grazing a unit-sized floor whose node also
+    //   held a triangle 900 units away lost 104 of 100,000 hits;
+    // - on the scale of the ray's distance, 3 * 2^-24 of its origin, as far as
+    //   half a step goes: of 1.2 million hits at edges from 1000 units away,
+    //   in the same scene, none is lost, against 68 without it and 38 with a
+    //   power-of-two step.
+    // On the scene of a million triangles rays visit 0.02% more nodes (camera
+    // rays 13.053 -> 13.055, bounce 22.709 -> 22.716, shadow 13.668 -> 13.670).
+    // A margin of half a step at every node: 0.4%, and a 256x256 frame 1.1%
+    // longer.
+    void quantise(BvhNode& nd, const Box* box, const int32_t* child, int cnt) const {
         bool used[4];
         for (int k = 0; k < 4; ++k) used[k] = k < cnt && child[k] != ~0;
         for (int a = 0; a < 3; ++a) {
@@ -408,7 +415,9 @@ struct Collapser {
                     hi = std::max(hi, box[k].hi[a]);
                 }
             if (!(lo <= hi)) lo = hi = 0.0f;  // no used child (cannot happen for a built tree)
-            const double m = std::ldexp(std::max({(double)hi - (double)lo, std::fabs((double)lo), std::fabs((double)hi)}), -21);
+            const double ext = (double)hi - (double)lo;
+            const double m = std::ldexp(std::max({ext, std::fabs((double)lo), std::fabs((double)hi)}), -21) +
+                             std::min(std::ldexp((double)reach, -20), ext / 510.0);
             const float org = down((double)lo - m);
             const double s = grid_step((double)hi + m - (double)org);
             nd.org[a] = org;
@@ -550,7 +559,9 @@ vgi_status build_scene_host(const vgi_scene_desc* desc, HostScene& hs) {
     }
     if (b.max_depth + 1 > kBvhMaxDepth)
         return set_error(VGI_E_UNSUPPORTED, "vgi_scene_create: BVH depth %d exceeds %d", b.max_depth + 1, kBvhMaxDepth);
-    Collapser c4{b.nodes, {}, 0, {}};
+    float reach = 0.0f;
+    for (int a = 0; a < 3; ++a) reach = std::max({reach, std::fabs(root_box.lo[a]), std::fabs(root_box.hi[a])});
+    Collapser c4{b.nodes, reach, {}, 0, {}};
     c4.plan();
     c4.out.reserve(b.nodes.size() / 2 + 1);
     root = c4.emit(root, 0);

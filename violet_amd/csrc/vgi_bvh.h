@@ -18,14 +18,14 @@
  *   tris  : leaf-ordered triangles as {v0, e1 = v1-v0, e2 = v2-v0} (3 x
  *           float4, 48 bytes); v0.w carries the scene triangle id.
  * Child boxes are padded, by 2^-16 of the child's coordinates (at least of 1)
- * and 2^-21 of the node's (vgi_bvh.cpp), so that neither the rounding of the
- * slab test (slab_q in vgi_traverse.h) nor that of the intersection routine
- * prunes a triangle that the routine accepts: the closest hit (smallest t,
- * ties to the lowest triangle id) equals a brute-force loop over all
- * triangles.  Both roundings also grow with the distance to the ray's origin,
- * which no stored box can cover: rays that start 300 units and more from
- * geometry of a unit's size near the scene's origin can lose a grazing hit
- * (about 70 of a million such rays, aimed at edges from 1000 units).
+ * and on the scales of their node and scene (quantise in vgi_bvh.cpp), so that
+ * neither the rounding of the slab test (slab_q in vgi_traverse.h) nor that of
+ * the intersection routine prunes a triangle that the routine accepts: the
+ * closest hit (smallest t, ties to the lowest triangle id) equals a brute-force
+ * loop over all triangles.  Both roundings also grow with the distance to the
+ * ray's origin, which no stored box bounds: of 1.2 million hits aimed at the
+ * edges of geometry of a unit's size near the origin of a scene of 900 units,
+ * none is lost from 1000 units away, 99 from 3000 and 567 from 10,000.
  *
  * Hit semantics follow violet: opaque, two-sided, t in [tmin, tmax];
  * shadow rays accept the first hit (RAY_FLAG_ACCEPT_FIRST_HIT_AND_END_SEARCH).

@@ -115,12 +115,13 @@ struct NodePlanes {
 // plane = org + q * step, the distance errs by at most u * extent (rounding
 // of a) + 2 u |org - o| (of the difference and its product) + u |plane - o|
 // (of the sum), in all 2 u extent + 3 u (|org| + |o|), besides the relative
-// error of idir that all planes of the axis share.  The node's grid boxes
-// hold 8 u max(extent, |org|) beyond the padded ones (quantise); the rest, up
-// to 3 u |o|, is the padding's to cover (at least 256 u): it does for origins
-// within 85 units, and 85 times the child's own distance from the scene's
-// origin.  An unused child (lo = 255, hi = 0) has its near plane beyond its
-// far one on every axis.
+// error of idir that all planes of the axis share.  Beyond the padded boxes
+// the node's grid boxes hold 8 u max(extent, |org|), more than the node's part
+// of that, and 16 u times the scene's reach or half a step (quantise).  So the
+// rest, up to 3 u |o|, is covered for origins within five times the reach at
+// nodes of a 2000th of it and more, and by the padding (at least 256 u) for
+// those within 85 units.  An unused child (lo = 255, hi = 0) has its near plane
+// beyond its far one on every axis.
 template <int k>
 __device__ __forceinline__ void slab_q(f3 a, f3 b, const NodePlanes& p, float tmin, float tmax, float& tn, float& tf) {
     const float tnx = __builtin_fmaf(qline<k>(p.nx01, p.nx23), a.x, b.x);

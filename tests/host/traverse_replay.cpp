@@ -200,7 +200,7 @@ void run_wave(const HostScene& s, std::vector<Lane>& w, Totals& totals, bool bou
                     l.p -= kStackStride;
                 }
             }
-            if (deep)
+            if (deep && (!kAny || n_leaf == 0))
                 for (Lane& l : w)
                     if (waits(l)) {
                         l.spilled -= kSpillEntries;

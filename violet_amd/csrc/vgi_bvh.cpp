@@ -12,8 +12,8 @@
  * children's padded boxes on an 8-bit grid spanning them (vgi_bvh.h).
  *
  * Against 32 bins, opening the largest child first and a power-of-two grid
- * step, rays on the 1M-triangle scene visit 7-9% fewer nodes (primary 14.3 ->
- * 13.0, bounce 19.7 -> 18.3, shadow 15.2 -> 14.2), and the tree has 20% fewer
+ * step, rays on the 1M-triangle scene visit 8-17% fewer nodes (camera 14.3 ->
+ * 13.1, bounce 24.7 -> 22.7, shadow 16.5 -> 13.7), and the tree has 20% fewer
  * of them.  Subtrees build on several threads; the tree does not depend on
  * how many.
  */

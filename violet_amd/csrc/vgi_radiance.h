@@ -291,7 +291,7 @@ __device__ __forceinline__ RadianceTraceResult trace_radiance(const TraceRes& rt
     SurfaceHit sh = shade_hit(rt.scene, hit, d);
     // A surface that faces away from the sun gets no light from it whether or
     // not something is in between (a finite BRDF and sun times a cosine of
-    // zero): no ray.  1080p frame 1591 -> 1577 us.
+    // zero): no ray.  1080p frame 1588 -> 1581 us, lit 803x451 520 -> 516 us.
     bool sun_visible = false;
     const f3 si = xyz(fp.sun_inten);
     const bool away = !(dot3(sh.normal, xyz(fp.sun_dir)) > 0.0f) && fabsf(si.x) + fabsf(si.y) + fabsf(si.z) < INFINITY;

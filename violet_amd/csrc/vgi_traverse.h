@@ -194,13 +194,13 @@ __device__ __forceinline__ bool closer_hit(f3 o, f3 d, Vf4 v0, Vf4 e1v, Vf4 e2v,
 // kCount: the instrumented build (traversal statistics) that adds this ray's
 // node and triangle counts to s.counters.
 //
-// What bounds it: vector instruction issue (the VALU is busy about 90% of
-// the cycles), then the round trip of each node.  So the wave steps through
-// nodes without a branch per child: a step tests four boxes, sorts them,
-// writes all four links to the stack (far to near, missed children last,
-// above the new top) and pops its next two entries in one LDS read; the
-// second one serves if the first is a leaf that is set aside.  A sentinel
-// under the stack ends the ray without a test for an empty stack.
+// What bounds it: vector instruction issue (while the chip is full), then the
+// round trip of each node.  So the wave steps through nodes without a branch
+// per child: a step tests four boxes, sorts them, writes all four links to the
+// stack (far to near, missed children last, above the new top) and pops its
+// next two entries in one LDS read; the second one serves if the first is a
+// leaf that is set aside.  A sentinel under the stack ends the ray without a
+// test for an empty stack.
 //
 // A lane sets aside the first leaf it reaches and goes on down the tree.
 // The wave takes a node step as long as at least two lanes want one (at a
@@ -219,9 +219,11 @@ __device__ __forceinline__ bool closer_hit(f3 o, f3 d, Vf4 v0, Vf4 e1v, Vf4 e2v,
 // -> 367 us.  A look at every node step instead costs small frames 0.4%.
 // Any-hit rays end early and gain nothing by it (33 -> 31 us); they wait.
 //
-// 1M bounce rays on 1M triangles: 324 -> 241 us; the 1080p sampling and
-// spatial passes 1210 -> 995 us; a 1080p frame 1951 -> 1687 us, a 256x256 one
-// 617 -> 493 us.  6 or 7 resident waves per SIMD instead of 8: within 3%.
+// Against a step with branches per child and the wait for a leaf in every
+// lane: 1M bounce rays on 1M triangles 324 -> 241 us (226 with the present
+// tree); the 1080p sampling and spatial passes 1210 -> 995 us; a 1080p frame
+// 1951 -> 1687 us, a 256x256 one 617 -> 493 us.  6 or 7 resident waves per SIMD
+// instead of 8: within 3%.
 template <bool kAnyHit, bool kCount = false>
 __device__ __forceinline__ Hit traverse(const SceneView& s, f3 o, f3 d, float tmin, float tmax, LdsStack stack) {
     const RayInv r = make_ray(o, d);
